@@ -168,9 +168,12 @@ using GraphCacheHip = GraphCache<GraphPayload>;
 
 // Scratch of the Earth / Moon finder.
 struct CCWork {
-    DevBuf<int> counts, starts, cellhash, sorted, block_sums, parent, size, mcounts;
-    DevBuf<unsigned long long> best;
+    DevBuf<int> counts, starts, cellhash, block_sums, parent, size, mcounts;
+    DevBuf<float4> spos;
+    DevBuf<CCTop> top;  // the blocks' two largest groups, then the whole's
     DevBuf<double> moments;
+    DevBuf<gi_earth_moon> result;
+    gi_earth_moon* host = nullptr;  // pinned: the call's one copy back
 };
 
 struct DevCtx {
@@ -1858,97 +1861,41 @@ int gi_find_earth_moon(const gi_float4* pos, const gi_float4* vel, int n, int nf
     if ((m + 1023) / 1024 > 4096) return set_error(GI_E_TOO_LARGE, "gi_find_earth_moon: n too large (%d)", n);
     const int nbs = nblk(m, 1024);
     if ((rc = w.counts.ensure(m + 1)) || (rc = w.starts.ensure(m + 2)) || (rc = w.cellhash.ensure(n)) ||
-        (rc = w.sorted.ensure(n)) || (rc = w.block_sums.ensure(nbs + 8)) || (rc = w.parent.ensure(n)) ||
-        (rc = w.size.ensure(n + 1)) || (rc = w.best.ensure(2)))
+        (rc = w.spos.ensure(n)) || (rc = w.block_sums.ensure(nbs + 8)) || (rc = w.parent.ensure(n)) ||
+        (rc = w.size.ensure(n + 1)) || (rc = w.top.ensure(kCCTopBlocks + 1)) || (rc = w.result.ensure(1)))
         return rc;
+    const int nb = std::min(1024, nblk(n, kCCBlock));
+    if ((rc = w.moments.ensure((size_t)nb * kCCClasses * kCCMoments)) ||
+        (rc = w.mcounts.ensure((size_t)nb * kCCCounts)))
+        return rc;
+    if (!w.host) GI_HIP(hipHostMalloc((void**)&w.host, sizeof(gi_earth_moon), hipHostMallocDefault));
     // cells a sixteenth larger than touch: a touching pair is never two cells apart
     const double inv_c = 1.0 / ((double)touch * 1.0625);
     const float4* P = (const float4*)pos;
     hipLaunchKernelGGL(k_fill_int, dim3(nblk(m, 256)), dim3(256), 0, st, w.counts.p, (int)m, 0);
     hipLaunchKernelGGL(k_cc_count, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, inv_c, m - 1, w.counts.p,
-                       w.cellhash.p);
+                       w.cellhash.p, w.size.p);
     hipLaunchKernelGGL(k_scan_blocks, dim3(nbs), dim3(256), 0, st, w.counts.p, (int)m, w.starts.p, w.block_sums.p);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, st, w.block_sums.p, nbs, w.starts.p + m);
     hipLaunchKernelGGL(k_scan_add, dim3(nblk(m, 256)), dim3(256), 0, st, w.starts.p, (int)m, w.block_sums.p);
-    hipLaunchKernelGGL(k_grid_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, n, w.cellhash.p, w.starts.p,
-                       w.counts.p, w.sorted.p);
-    hipLaunchKernelGGL(k_cc_init, dim3(nblk(n, 256)), dim3(256), 0, st, w.parent.p, w.size.p, n);
-    hipLaunchKernelGGL(k_cc_union, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, inv_c, m - 1, touch, w.starts.p,
-                       w.sorted.p, w.parent.p);
-    hipLaunchKernelGGL(k_cc_compress, dim3(nblk(n, 256)), dim3(256), 0, st, w.parent.p, w.size.p, n);
-    const unsigned long long zero[2] = {0ull, 0ull};
-    GI_HIP(hipMemcpyAsync(w.best.p, zero, sizeof zero, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_cc_top, dim3(nblk(n, 256)), dim3(256), 0, st, w.size.p, n, -1, w.best.p);
+    hipLaunchKernelGGL(k_cc_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, w.cellhash.p, w.starts.p, w.counts.p,
+                       w.spos.p);
+    hipLaunchKernelGGL(k_cc_local, dim3(nblk(n, kCCLocal)), dim3(kCCLocal), 0, st, w.spos.p, n, inv_c, m - 1, touch,
+                       w.starts.p, w.parent.p);
+    hipLaunchKernelGGL(k_cc_union, dim3(nblk(n, kCCUnionPer)), dim3(64 * kCCUnionWaves), 0, st, w.spos.p, n, inv_c,
+                       m - 1, touch, w.starts.p, w.parent.p);
+    hipLaunchKernelGGL(k_cc_compress, dim3(nblk(n, kCCCompressThreads)), dim3(kCCCompressThreads), 0, st, w.parent.p,
+                       w.size.p, n, group);
+    const int nt = std::min(kCCTopBlocks, nblk(n, 256));
+    CCTop* best = w.top.p + kCCTopBlocks;
+    hipLaunchKernelGGL(k_cc_top, dim3(nt), dim3(256), 0, st, w.size.p, n, w.top.p);
+    hipLaunchKernelGGL(k_cc_moments, dim3(nb), dim3(kCCBlock), 0, st, P, (const float4*)vel, n, w.parent.p, w.top.p,
+                       nt, best, nfe1, nfe2, nsi1, mass_fe, mass_si, w.moments.p, w.mcounts.p);
+    hipLaunchKernelGGL(k_cc_final, dim3(1), dim3(32 * kCCFinalSegs), 0, st, w.moments.p, w.mcounts.p, nb, best, w.result.p);
     GI_HIP(hipGetLastError());
-    unsigned long long best[2];
-    GI_HIP(hipMemcpyAsync(best, w.best.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+    GI_HIP(hipMemcpyAsync(w.host, w.result.p, sizeof(gi_earth_moon), hipMemcpyDeviceToHost, st));
     GI_HIP(hipStreamSynchronize(st));
-    const int earth = (int)~(unsigned)(best[0] & 0xffffffffull);
-    hipLaunchKernelGGL(k_cc_top, dim3(nblk(n, 256)), dim3(256), 0, st, w.size.p, n, earth, w.best.p + 1);
-    GI_HIP(hipGetLastError());
-    GI_HIP(hipMemcpyAsync(best + 1, w.best.p + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    GI_HIP(hipStreamSynchronize(st));
-    const int moon = best[1] ? (int)~(unsigned)(best[1] & 0xffffffffull) : -1;
-    // moments of the system, the Earth and the Moon
-    const int nb = std::min(1024, nblk(n, kCCBlock));
-    if ((rc = w.moments.ensure((size_t)nb * kCCClasses * kCCMoments)) ||
-        (rc = w.mcounts.ensure((size_t)nb * kCCCounts)))
-        return rc;
-    hipLaunchKernelGGL(k_cc_moments, dim3(nb), dim3(kCCBlock), 0, st, P, (const float4*)vel, n, w.parent.p, earth,
-                       moon, nfe1, nfe2, nsi1, mass_fe, mass_si, w.moments.p, w.mcounts.p);
-    GI_HIP(hipGetLastError());
-    std::vector<double> mom((size_t)nb * kCCClasses * kCCMoments);
-    std::vector<int> cnt((size_t)nb * kCCCounts);
-    std::vector<int> sizes(n);
-    GI_HIP(hipMemcpyAsync(mom.data(), w.moments.p, mom.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    GI_HIP(hipMemcpyAsync(cnt.data(), w.mcounts.p, cnt.size() * sizeof(int), hipMemcpyDeviceToHost, st));
-    GI_HIP(hipMemcpyAsync(sizes.data(), w.size.p, sizes.size() * sizeof(int), hipMemcpyDeviceToHost, st));
-    if (group) GI_HIP(hipMemcpyAsync(group, w.parent.p, (size_t)n * sizeof(int), hipMemcpyDeviceToDevice, st));
-    GI_HIP(hipStreamSynchronize(st));
-    // sums over blocks in block order; scope 1 (Earth-Moon) = Earth + Moon
-    double M[4][kCCMoments] = {};
-    for (int b = 0; b < nb; ++b)
-        for (int c = 0; c < kCCClasses; ++c)
-            for (int k = 0; k < kCCMoments; ++k)
-                M[c == 0 ? 0 : c + 1][k] += mom[((size_t)b * kCCClasses + c) * kCCMoments + k];
-    for (int k = 0; k < kCCMoments; ++k) M[1][k] = M[2][k] + M[3][k];
-    std::memset(out, 0, sizeof *out);
-    int c8[kCCCounts] = {};
-    for (int b = 0; b < nb; ++b)
-        for (int k = 0; k < kCCCounts; ++k) c8[k] += cnt[(size_t)b * kCCCounts + k];
-    out->n_groups = 0;
-    for (int i = 0; i < n; ++i) out->n_groups += sizes[i] > 0;
-    out->earth_id = earth;
-    out->moon_id = moon;
-    out->earth_count = sizes[earth];
-    out->moon_count = moon >= 0 ? sizes[moon] : 0;
-    out->earth_fe1 = c8[0];
-    out->earth_fe2 = c8[1];
-    out->earth_si1 = c8[2];
-    out->earth_si2 = c8[3];
-    out->moon_fe1 = c8[4];
-    out->moon_fe2 = c8[5];
-    out->moon_si1 = c8[6];
-    out->moon_si2 = c8[7];
-    for (int s = 0; s < 4; ++s) {
-        const double* a = M[s];
-        const double mass = a[0];
-        out->mass[s] = mass;
-        for (int d = 0; d < 3; ++d) {
-            out->com[s][d] = a[1 + d] / mass;  // 0/0 = NaN for an empty scope, as the reference divides
-            out->vel[s][d] = a[4 + d] / mass;
-        }
-        // L about the scope's centre of mass relative to its mean velocity:
-        // sum m x cross v - (sum m x) cross (sum m v) / M
-        const double* X = a + 1;
-        const double* Pm = a + 4;
-        const double cx = (X[1] * Pm[2] - X[2] * Pm[1]) / mass;
-        const double cy = (X[2] * Pm[0] - X[0] * Pm[2]) / mass;
-        const double cz = (X[0] * Pm[1] - X[1] * Pm[0]) / mass;
-        out->angmom[s][0] = a[7] - cx;
-        out->angmom[s][1] = a[8] - cy;
-        out->angmom[s][2] = a[9] - cz;
-    }
+    *out = *w.host;
     return 0;
 }
 
