@@ -181,7 +181,7 @@ struct DevCtx {
     Workspace ws;
     CCWork cc;
     DevBuf<double> rc_blocks, rc_sums;
-    DevBuf<float> rc_shift;  // the reference-float recenter's six shifts
+    DevBuf<unsigned char> rc_ref;  // the reference-float recenter's scratch (RcWork)
     hipStream_t capture_stream = nullptr;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     // side stream of a force evaluation (default priority): the contact grid
@@ -1237,16 +1237,49 @@ static int launch_recenter(DevCtx* ctx, float4* pos, float4* vel, int n, int nfe
     return 0;
 }
 
-// The reference's float recenter (k_recenter_ref_sum: its host sums in its
-// order, one workgroup) and the shift of every particle.
+// The reference-float recenter's scratch for n particles, laid out in one
+// buffer of the device's context.  Windows of 64 particles, doubled until
+// one workgroup joins a chain's runs.
+static int recenter_ref_scratch(DevCtx* ctx, int n, RcWork* wk) {
+    wk->window = 64;
+    while (nblk(n, wk->window) > kRcMaxRuns) wk->window *= 2;
+    const size_t w = wk->nwin = nblk(n, wk->window);
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at = (at + bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t runs = take(kRcChains * w * kRcStarts * sizeof(RcRun)), sums = take(kRcChains * w * sizeof(double)),
+                 bound = take(kRcChains * (w + 1) * sizeof(int)), guess = take(kRcChains * w * sizeof(float)),
+                 total = take(kRcChains * sizeof(float));
+    int rc = ctx->rc_ref.ensure(at);
+    if (rc) return rc;
+    unsigned char* p = ctx->rc_ref.p;
+    wk->runs = (RcRun*)(p + runs);
+    wk->sums = (double*)(p + sums);
+    wk->bound = (int*)(p + bound);
+    wk->guess = (float*)(p + guess);
+    wk->total = (float*)(p + total);
+    return 0;
+}
+
+// The reference's float recenter (its host sums, rounding for rounding) and
+// the shift of every particle.
 static int launch_recenter_ref(DevCtx* ctx, float4* pos, float4* vel, int n, int nfe, double mfe, double msi,
                                const float* tc, const float* tv, hipStream_t st) {
+    RcWork wk;
     int rc;
-    if ((rc = ctx->rc_shift.ensure(8))) return rc;
-    hipLaunchKernelGGL(k_recenter_ref_sum, dim3(1), dim3(256), 0, st, (const float4*)pos, (const float4*)vel, n, nfe,
-                       mfe, msi, tc[0], tc[1], tc[2], tv[0], tv[1], tv[2], ctx->rc_shift.p);
+    if ((rc = recenter_ref_scratch(ctx, n, &wk))) return rc;
+    const float4 *P = pos, *V = vel;
+    const dim3 wgrid(nblk(wk.nwin, kRcWindowWaves)), wblock(64 * kRcWindowWaves);
+    hipLaunchKernelGGL(k_rc_window_sums, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
+    hipLaunchKernelGGL(k_rc_bounds, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
+    hipLaunchKernelGGL(k_rc_runs, dim3(nblk((long long)kRcChains * wk.nwin * kRcStarts, 256)), dim3(256), 0, st, P, V,
+                       nfe, mfe, msi, wk);
+    hipLaunchKernelGGL(k_rc_join, dim3(kRcChains), dim3(kRcJoinThreads), 0, st, P, V, nfe, mfe, msi, wk);
     hipLaunchKernelGGL(k_recenter_ref_apply, dim3(nblk(n, 256)), dim3(256), 0, st, pos, vel, n,
-                       (const float*)ctx->rc_shift.p);
+                       (const float*)wk.total, tc[0], tc[1], tc[2], tv[0], tv[1], tv[2]);
     GI_HIP(hipGetLastError());
     return 0;
 }
@@ -2003,8 +2036,9 @@ static int impact_steps_impl(gi_float4* pos, gi_float4* vel, gi_float4* force, i
                 key_append(k2, rs.tcf[a]);
                 key_append(k2, rs.tvf[a]);
             }
-            if ((rc = ctx->rc_shift.ensure(8))) return rc;
-            key_append(k2, ctx->rc_shift.p);
+            RcWork wk;
+            if ((rc = recenter_ref_scratch(ctx, n, &wk))) return rc;
+            key_append(k2, ctx->rc_ref.p);
             rc = get_graph(ctx, ctx->graphs, k2, ctx->ws.generation,
                            [&](hipStream_t cs) -> int {
                                return launch_recenter_ref(ctx, P, V, n, fc->NFe, rs.mass_fe, rs.mass_si, rs.tcf,

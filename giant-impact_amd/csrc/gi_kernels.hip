@@ -1703,58 +1703,355 @@ __global__ void k_recenter_apply(float4* __restrict__ pos, float4* __restrict__ 
 // 388-417) accumulate in float on the host, particle by particle in index
 // order: acc = float(double(acc) + double(x) * m) with m the double element
 // mass (iron for i < nfe), and the mass the same way with x = 1.  Each of
-// those seven sums is one sequential chain, so one workgroup stages the
-// particles through LDS a tile at a time (coalesced loads by all its lanes)
-// and seven lanes of its first wavefront run the chains side by side.  The
-// result is written as the six float shifts target - mean that every
-// particle then adds (k_recenter_ref_apply): bitwise the reference's host
-// loop.
-constexpr int kRecenterTile = 1024;
+// those seven sums ("chains") is n dependent roundings.
+//
+// Taken one after another they cost 52 ns each on the device (3.4 ms at
+// N = 65,536).  They need not be: a step a -> float(double(a) + t) commutes
+// with a shift d of a whenever d is a multiple of two float ulps of the
+// binade the step's sum lies in and neither the sum nor the shifted sum
+// leaves that binade (then both roundings, to double and to float, act on
+// the same grid, and d keeps the parity that ties look at).  So a run of
+// steps can be taken from a guessed start g, and holds for the true start a
+// too if d = a - g is such a multiple for the run's largest binade and |d| is
+// smaller than every sum's distance from its binade's ends: its end is then
+// the guess's end plus d, exactly.
+//   k_rc_window_sums   FP64 sums of windows of the chain;
+//   k_rc_bounds        cuts the chain in each window where the FP64 prefix is
+//                      largest (the coarsest grid there, so few residues of
+//                      the start matter) and guesses the start from it;
+//   k_rc_runs          every run from 16 starts, one float ulp apart (they
+//                      cover every residue up to 8 ulps), with its largest
+//                      binade and least distance;
+//   k_rc_join          one workgroup per chain: runs joined in groups of 16
+//                      from the group's 16 starts side by side, then the
+//                      groups in order from the true start; where the
+//                      conditions do not hold, run by run, and a run that
+//                      does not hold is taken step by step.  No result
+//                      depends on a guess: a guess only decides which way it
+//                      is reached.
+// Bound by the join's chain of dependent FP64 operations.  The impact states
+// need 0 to 9 of 1,024 runs step by step.  N = 65,536: 122 us a call (sums
+// 5 us, bounds 18, runs 23, join 50 to 110, apply 5) against 3,404 step by
+// step; windows of 128 took 135.
+constexpr int kRcChains = 7;
+constexpr int kRcStarts = 16;
+constexpr int kRcGroup = 16;     // runs per group
+constexpr int kRcMaxRuns = 1024;
+constexpr float kRcRoom = 1.0e30f;  // no step yet
+constexpr int kRcJoinThreads = kRcMaxRuns / kRcGroup * kRcStarts;
+static_assert(kRcJoinThreads <= 1024, "one workgroup joins a chain");
 
-__global__ __launch_bounds__(256) void k_recenter_ref_sum(const float4* __restrict__ pos,
-                                                          const float4* __restrict__ vel, int n, int nfe,
-                                                          double mass_fe, double mass_si, float tcx, float tcy,
-                                                          float tcz, float tvx, float tvy, float tvz,
-                                                          float* __restrict__ shift) {
-    __shared__ float tile[6][kRecenterTile];
-    const int lane = threadIdx.x;
-    float acc = 0.0f;  // lanes 0..5: sum m * (x, y, z, vx, vy, vz); lane 6: sum m
-    for (int t0 = 0; t0 < n; t0 += kRecenterTile) {
-        const int cnt = min(kRecenterTile, n - t0);
-        __syncthreads();  // the previous tile's chains are done
-        for (int k = lane; k < cnt; k += blockDim.x) {
-            const float4 p = pos[t0 + k];
-            const float4 v = vel[t0 + k];
-            tile[0][k] = p.x;
-            tile[1][k] = p.y;
-            tile[2][k] = p.z;
-            tile[3][k] = v.x;
-            tile[4][k] = v.y;
-            tile[5][k] = v.z;
-        }
-        __syncthreads();
-        if (lane < 7) {
-            for (int k = 0; k < cnt; ++k) {
-                const double m = t0 + k < nfe ? mass_fe : mass_si;
-                const double x = lane < 6 ? (double)tile[lane][k] : 1.0;
-                acc = (float)((double)acc + x * m);
-            }
-        }
+// A run from one start: its end, the least distance of a sum from its
+// binade's ends (negative: never shift this run) and the largest binade.
+struct __align__(16) RcRun {
+    float end;
+    int binade;
+    float room;
+    int pad;
+};
+
+// Scratch of one recenter over runs of `window` particles.
+struct RcWork {
+    double* sums;   // [kRcChains][nwin]
+    int* bound;     // [kRcChains][nwin + 1]
+    float* guess;   // [kRcChains][nwin]
+    RcRun* runs;    // [kRcChains][nwin][kRcStarts]
+    float* total;   // [kRcChains]
+    int window, nwin;
+};
+
+// Term k of chain c: x, y, z, vx, vy, vz, 1 times the element's mass.
+__device__ __forceinline__ float rc_value(const float4* __restrict__ pos, const float4* __restrict__ vel, int c,
+                                          int k) {
+    if (c == 6) return 1.0f;
+    return reinterpret_cast<const float*>(c < 3 ? pos : vel)[4 * (size_t)k + (c < 3 ? c : c - 3)];
+}
+
+__device__ __forceinline__ void rc_terms(const float4* __restrict__ pos, const float4* __restrict__ vel, int k,
+                                         double m, double (&t)[kRcChains]) {
+    const float4 p = pos[k], v = vel[k];
+    t[0] = (double)p.x * m;
+    t[1] = (double)p.y * m;
+    t[2] = (double)p.z * m;
+    t[3] = (double)v.x * m;
+    t[4] = (double)v.y * m;
+    t[5] = (double)v.z * m;
+    t[6] = m;
+}
+
+constexpr int kRcWindowWaves = 4;  // windows per workgroup, a wavefront each
+
+// End of window w (also where the particle count is near the int range's end).
+__device__ __forceinline__ int rc_window_end(const RcWork& wk, int w, int n) {
+    return (int)min((long long)(w + 1) * wk.window, (long long)n);
+}
+
+__global__ __launch_bounds__(64 * kRcWindowWaves) void k_rc_window_sums(const float4* __restrict__ pos,
+                                                                       const float4* __restrict__ vel, int n,
+                                                                       int nfe, double mass_fe, double mass_si,
+                                                                       RcWork wk) {
+    const int lane = threadIdx.x & 63;
+    const int w = blockIdx.x * kRcWindowWaves + (threadIdx.x >> 6);
+    if (w >= wk.nwin) return;
+    double s[kRcChains] = {};
+    const int e = rc_window_end(wk, w, n);
+    for (long long k = (long long)w * wk.window + lane; k < e; k += 64) {
+        double t[kRcChains];
+        rc_terms(pos, vel, (int)k, k < nfe ? mass_fe : mass_si, t);
+#pragma unroll
+        for (int c = 0; c < kRcChains; ++c) s[c] += t[c];
     }
-    __shared__ float sums[7];
-    if (lane < 7) sums[lane] = acc;
-    __syncthreads();
-    if (lane < 6) {
-        // centerOfMass.x /= totalMass in float: the double quotient rounded
-        // once to float is the correctly rounded float quotient (53 >= 2*24+2).
-        const float mean = (float)((double)sums[lane] / (double)sums[6]);
-        const float target = lane == 0 ? tcx : lane == 1 ? tcy : lane == 2 ? tcz : lane == 3 ? tvx : lane == 4 ? tvy : tvz;
-        shift[lane] = target - mean;
+#pragma unroll
+    for (int c = 0; c < kRcChains; ++c) {
+#pragma unroll
+        for (int m = 32; m; m >>= 1) s[c] += __shfl_xor(s[c], m);
+        if (lane == c) wk.sums[c * wk.nwin + w] = s[c];
     }
 }
 
+__global__ __launch_bounds__(64 * kRcWindowWaves) void k_rc_bounds(const float4* __restrict__ pos,
+                                                                  const float4* __restrict__ vel, int n, int nfe,
+                                                                  double mass_fe, double mass_si, RcWork wk) {
+    const int lane = threadIdx.x & 63;
+    const int w = blockIdx.x * kRcWindowWaves + (threadIdx.x >> 6);
+    if (w >= wk.nwin) return;
+    // the prefix before the window
+    double p[kRcChains] = {};
+    for (int k = lane; k < w; k += 64)
+#pragma unroll
+        for (int c = 0; c < kRcChains; ++c) p[c] += wk.sums[c * wk.nwin + k];
+    // this lane's share of the window: consecutive elements
+    const int per = wk.window / 64;
+    const int end = rc_window_end(wk, w, n);
+    const int k0 = (int)min((long long)w * wk.window + lane * per, (long long)end), k1 = min((long long)k0 + per, (long long)end);
+    double own[kRcChains] = {};
+    for (int k = k0; k < k1; ++k) {
+        double t[kRcChains];
+        rc_terms(pos, vel, k, k < nfe ? mass_fe : mass_si, t);
+#pragma unroll
+        for (int c = 0; c < kRcChains; ++c) own[c] += t[c];
+    }
+#pragma unroll
+    for (int c = 0; c < kRcChains; ++c) {
+#pragma unroll
+        for (int m = 32; m; m >>= 1) p[c] += __shfl_xor(p[c], m);
+        double before = own[c];
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const double o = __shfl_up(before, m);
+            if (lane >= m) before += o;
+        }
+        p[c] += before - own[c];
+    }
+    // the place of the largest prefix in the window
+    double best[kRcChains], at[kRcChains];
+    int place[kRcChains];
+#pragma unroll
+    for (int c = 0; c < kRcChains; ++c) {
+        best[c] = -1.0;
+        at[c] = 0.0;
+        place[c] = 0x7fffffff;
+    }
+    for (int k = k0; k < k1; ++k) {
+        double t[kRcChains];
+        rc_terms(pos, vel, k, k < nfe ? mass_fe : mass_si, t);
+#pragma unroll
+        for (int c = 0; c < kRcChains; ++c) {
+            p[c] += t[c];
+            if (fabs(p[c]) > best[c]) {
+                best[c] = fabs(p[c]);
+                at[c] = p[c];
+                place[c] = k + 1;
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < kRcChains; ++c) {
+#pragma unroll
+        for (int m = 32; m; m >>= 1) {
+            const double ob = __shfl_xor(best[c], m), oa = __shfl_xor(at[c], m);
+            const int op = __shfl_xor(place[c], m);
+            if (ob > best[c] || (ob == best[c] && op < place[c])) {
+                best[c] = ob;
+                at[c] = oa;
+                place[c] = op;
+            }
+        }
+        if (lane == 0) {
+            int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
+            float* __restrict__ guess = wk.guess + c * wk.nwin;
+            if (w == 0) {
+                bound[0] = 0;
+                guess[0] = 0.0f;
+            }
+            const bool last = w + 1 == wk.nwin;
+            // a window of NaNs has no largest prefix: cut at its end
+            bound[w + 1] = last ? n : (best[c] >= 0.0 ? place[c] : end);
+            if (!last) guess[w + 1] = (float)at[c];
+        }
+    }
+}
+
+// Start j of a run guessed to begin at g: j float ulps of g's binade above g.
+__device__ __forceinline__ double rc_ulp(float g) {
+    const int e = (int)((__float_as_uint(g) >> 23) & 0xff);
+    // zero, denormal, infinite and NaN guesses have no ulp to step by
+    return e == 0 || e == 255 ? 0.0 : __longlong_as_double((long long)(e - 127 - 23 + 1023) << 52);
+}
+__device__ __forceinline__ float rc_start(float g, int j) { return (float)((double)g + (double)j * rc_ulp(g)); }
+
+// One step with term t = x * mass: the sum's rounding to float, its binade
+// and its distance from the binade's ends, rounded down to the sum's 21
+// leading bits.  A zero term changes nothing from any start.
+__device__ __forceinline__ void rc_step(float& a, float x, double t, int& binade, float& room) {
+    const double s = (double)a + t;
+    const int hi = __double2hiint(s) & 0x7fffffff;
+    const int e = hi >> 20;
+    const int m = hi & 0xfffff;
+    float r = __builtin_amdgcn_ldexpf((float)min(m, 0xfffff - m), e - 1023 - 20);
+    // well inside the float range only (not infinite or NaN)
+    if ((unsigned)(e - (1023 - 80)) > 160u) r = -1.0f;
+    if (x != 0.0f) {
+        binade = max(binade, e);
+        room = fminf(room, r);
+    }
+    a = (float)s;
+}
+
+__global__ __launch_bounds__(256) void k_rc_runs(const float4* __restrict__ pos, const float4* __restrict__ vel,
+                                                 int nfe, double mass_fe, double mass_si, RcWork wk) {
+    const int id = blockIdx.x * 256 + threadIdx.x;
+    const int j = id % kRcStarts, s = id / kRcStarts % wk.nwin, c = id / kRcStarts / wk.nwin;
+    if (c >= kRcChains) return;
+    const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
+    const int b = bound[s], e = bound[s + 1];
+    RcRun r{rc_start(wk.guess[c * wk.nwin + s], j), 0, kRcRoom, 0};
+    float x[8], nx[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = rc_value(pos, vel, c, min(b + u, e - 1));
+    for (int k = b; k < e; k += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) nx[u] = rc_value(pos, vel, c, min(k + 8 + u, e - 1));
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (k + u < e) rc_step(r.end, x[u], (double)x[u] * (k + u < nfe ? mass_fe : mass_si), r.binade, r.room);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = nx[u];
+    }
+    wk.runs[((size_t)c * wk.nwin + s) * kRcStarts + j] = r;
+}
+
+// The start of a run or group guessed at g that the true start `a` differs
+// from by a multiple of kRcStarts ulps, and that difference.
+struct RcShift {
+    int j;
+    double d;
+    bool exact;
+};
+__device__ __forceinline__ RcShift rc_shift(float a, float g) {
+    const int e = (int)((__float_as_uint(g) >> 23) & 0xff);
+    RcShift x{0, 0.0, false};
+    const double k = __builtin_amdgcn_ldexp((double)a - (double)g, 127 + 23 - e);  // in ulps of g
+    if (e != 0 && e != 255 && fabs(k) < 1.0e9) x.j = (int)rint(k) & (kRcStarts - 1);
+    const float s = rc_start(g, x.j);
+    x.d = (double)a - (double)s;
+    x.exact = (double)a - x.d == (double)s;
+    return x;
+}
+// Whether a run holds when its start is shifted by d.
+__device__ __forceinline__ bool rc_holds(const RcShift& x, int binade, float room) {
+    if (!x.exact) return false;
+    if (x.d == 0.0 || binade == 0) return true;  // binade 0: every term is zero
+    if (!(fabs(x.d) < (double)room)) return false;
+    const double k = __builtin_amdgcn_ldexp(x.d, 1023 + 22 - binade);  // in pairs of ulps
+    return k == rint(k);
+}
+__device__ __forceinline__ float rc_shifted(const RcRun& r, const RcShift& h) { return (float)((double)r.end + h.d); }
+
+__global__ __launch_bounds__(kRcJoinThreads) void k_rc_join(const float4* __restrict__ pos,
+                                                            const float4* __restrict__ vel, int nfe, double mass_fe,
+                                                            double mass_si, RcWork wk) {
+    __shared__ RcRun group[kRcJoinThreads];
+    __shared__ RcRun one[kRcGroup * kRcStarts];  // the runs of a group that does not hold
+    __shared__ float guess[kRcMaxRuns];
+    __shared__ double terms[64];
+    const int c = blockIdx.x;
+    const RcRun* __restrict__ runs = wk.runs + (size_t)c * wk.nwin * kRcStarts;
+    const int ngroups = (wk.nwin + kRcGroup - 1) / kRcGroup;
+    const int g = threadIdx.x / kRcStarts, j = threadIdx.x % kRcStarts;
+    for (int s = threadIdx.x; s < wk.nwin; s += kRcJoinThreads) guess[s] = wk.guess[c * wk.nwin + s];
+    __syncthreads();
+    if (g < ngroups) {
+        RcRun x{rc_start(guess[g * kRcGroup], j), 0, kRcRoom, 0};
+        for (int s = g * kRcGroup; s < min((g + 1) * kRcGroup, wk.nwin); ++s) {
+            const RcShift h = rc_shift(x.end, guess[s]);
+            const RcRun r = runs[s * kRcStarts + h.j];
+            if (!rc_holds(h, r.binade, r.room)) {
+                x.binade = -1;
+                break;
+            }
+            x.end = rc_shifted(r, h);
+            x.binade = max(x.binade, r.binade);
+            // rounded down: the least factor below 1 takes more than the
+            // subtraction's and the conversion's rounding
+            x.room = fminf(x.room, (float)(((double)r.room - fabs(h.d)) * (1.0 - 0x1p-20)));
+        }
+        group[threadIdx.x] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
+    float a = 0.0f;
+    for (int q = 0; q < ngroups; ++q) {
+        {
+            const RcShift h = rc_shift(a, guess[q * kRcGroup]);
+            const RcRun r = group[q * kRcStarts + h.j];
+            if (r.binade >= 0 && rc_holds(h, r.binade, r.room)) {
+                a = rc_shifted(r, h);
+                continue;
+            }
+        }
+        const int s0 = q * kRcGroup, s1 = min(s0 + kRcGroup, wk.nwin);
+        wave_lds_sync();
+        for (int k = lane; k < (s1 - s0) * kRcStarts; k += 64) one[k] = runs[s0 * kRcStarts + k];
+        const int edge = bound[min(s0 + lane, wk.nwin)];  // lanes 0..kRcGroup
+        wave_lds_sync();
+        for (int s = s0; s < s1; ++s) {
+            const RcShift h = rc_shift(a, guess[s]);
+            const RcRun r = one[(s - s0) * kRcStarts + h.j];
+            if (rc_holds(h, r.binade, r.room)) {
+                a = rc_shifted(r, h);
+                continue;
+            }
+            const int e = __shfl(edge, s + 1 - s0);
+            for (int k0 = __shfl(edge, s - s0); k0 < e; k0 += 64) {
+                wave_lds_sync();
+                const int k = min(k0 + lane, e - 1);
+                // past the run's end: -0 leaves every sum as it is
+                terms[lane] = k0 + lane < e ? (double)rc_value(pos, vel, c, k) * (k < nfe ? mass_fe : mass_si) : -0.0;
+                wave_lds_sync();
+#pragma unroll 8
+                for (int u = 0; u < 64; ++u) a = (float)((double)a + terms[u]);
+            }
+        }
+    }
+    if (lane == 0) wk.total[c] = a;
+}
+
 __global__ void k_recenter_ref_apply(float4* __restrict__ pos, float4* __restrict__ vel, int n,
-                                     const float* __restrict__ shift) {
+                                     const float* __restrict__ total, float tcx, float tcy, float tcz, float tvx,
+                                     float tvy, float tvz) {
+    __shared__ float shift[6];
+    const int lane = threadIdx.x;
+    if (lane < 6) {
+        // centerOfMass.x /= totalMass in float: the double quotient rounded
+        // once to float is the correctly rounded float quotient (53 >= 2*24+2).
+        const float mean = (float)((double)total[lane] / (double)total[6]);
+        const float target = lane == 0 ? tcx : lane == 1 ? tcy : lane == 2 ? tcz : lane == 3 ? tvx : lane == 4 ? tvy : tvz;
+        shift[lane] = target - mean;
+    }
+    __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4 p = pos[i];
