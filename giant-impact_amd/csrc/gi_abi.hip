@@ -574,7 +574,7 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
         for (size_t si = 0; si < sims.size(); ++si)
             if (sims[si].active)
                 for (int i0 = sims[si].start; i0 < sims[si].end; i0 += ib)
-                    p.dblocks.push_back(DirectBlock{(int)si, i0});
+                    p.dblocks.push_back(DirectBlock{(int)si, i0, sims[si].start, sims[si].fe_end, sims[si].end, 0, 0, 0});
         p.direct = true;
     }
     long long pbase = 0;
@@ -1049,18 +1049,26 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
     return 0;
 }
 
-template <bool POT, int MOVE>
-static void direct_kernel(int lanes, dim3 grid, dim3 block, hipStream_t st, const float4* pos, const float4* vel,
-                          const Workspace* ws, float4* force, double* pe, const FusedMove& mv) {
-    const DirectBlock* bl = ws->dblocks.p;
-    if (lanes == 8)
-        hipLaunchKernelGGL((k_direct<POT, 8, MOVE>), grid, block, 0, st, pos, vel, bl, ws->sims.p, force, pe, mv);
-    else if (lanes == 4)
-        hipLaunchKernelGGL((k_direct<POT, 4, MOVE>), grid, block, 0, st, pos, vel, bl, ws->sims.p, force, pe, mv);
-    else if (lanes == 2)
-        hipLaunchKernelGGL((k_direct<POT, 2, MOVE>), grid, block, 0, st, pos, vel, bl, ws->sims.p, force, pe, mv);
+// Wavefronts per workgroup of k_direct for n particles (of all simulations):
+// up to 2,048 particles there is a workgroup per CU at most, and 16
+// wavefronts shorten its chain (a step of N = 2,048 takes 9.8 us against 10.2
+// with 8); above, 8 leave room for the next workgroup beside the running ones
+// (N = 3,000 13.1 against 15.4 us, 4,096 15.2 against 17.9, 11,000 53 against
+// 69; four wavefronts were slower up to 8,192 and even above).
+constexpr long long kDirectWideMaxN = 2048;
+static int direct_waves(long long n) { return n <= kDirectWideMaxN ? 16 : 8; }
+
+// k_direct over a block table of 64 / lanes i-particles per entry.
+template <int MOVE>
+static void direct_kernel(int lanes, int waves, int nblocks, hipStream_t st, const float4* pos, const float4* vel,
+                          const DirectBlock* blocks, const SimDesc* sims, float4* force, const FusedMove& mv) {
+    int per_log2 = 0;
+    while ((kDirectI << per_log2) * lanes < 64) ++per_log2;
+    const dim3 grid((unsigned)nblocks << per_log2), block(64 * waves);
+    if (waves == 16)
+        hipLaunchKernelGGL((k_direct<MOVE, 16>), grid, block, 0, st, pos, vel, blocks, per_log2, sims, force, mv);
     else
-        hipLaunchKernelGGL((k_direct<POT, 1, MOVE>), grid, block, 0, st, pos, vel, bl, ws->sims.p, force, pe, mv);
+        hipLaunchKernelGGL((k_direct<MOVE, 8>), grid, block, 0, st, pos, vel, blocks, per_log2, sims, force, mv);
 }
 
 // The direct pass of the current plan: the force, or with pot the
@@ -1078,16 +1086,25 @@ static int launch_direct(DevCtx* ctx, Workspace* ws, const float4* pos, const fl
         GI_HIP(hipEventRecord(t2.a, st));
         GI_HIP(hipEventRecord(t0.a, st));
     }
-    const dim3 grid(nb), block(64 * kDirectWaves);
-    const int lanes = p.direct_lanes;
-    if (pot)
-        direct_kernel<true, 0>(lanes, grid, block, st, pos, vel, ws, nullptr, ws->pe.p, mv);
-    else if (move == 1)
-        direct_kernel<false, 1>(lanes, grid, block, st, pos, vel, ws, force, nullptr, mv);
-    else if (move == 2)
-        direct_kernel<false, 2>(lanes, grid, block, st, pos, vel, ws, force, nullptr, mv);
-    else
-        direct_kernel<false, 0>(lanes, grid, block, st, pos, vel, ws, force, nullptr, mv);
+    const int lanes = p.direct_lanes, waves = direct_waves(p.ntot);
+    const DirectBlock* bl = ws->dblocks.p;
+    if (pot) {
+        const dim3 grid(nb), block(64 * kDirectWaves);
+        if (lanes == 8)
+            hipLaunchKernelGGL(k_direct_potential<8>, grid, block, 0, st, pos, bl, ws->sims.p, ws->pe.p);
+        else if (lanes == 4)
+            hipLaunchKernelGGL(k_direct_potential<4>, grid, block, 0, st, pos, bl, ws->sims.p, ws->pe.p);
+        else if (lanes == 2)
+            hipLaunchKernelGGL(k_direct_potential<2>, grid, block, 0, st, pos, bl, ws->sims.p, ws->pe.p);
+        else
+            hipLaunchKernelGGL(k_direct_potential<1>, grid, block, 0, st, pos, bl, ws->sims.p, ws->pe.p);
+    } else if (move == 1) {
+        direct_kernel<1>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+    } else if (move == 2) {
+        direct_kernel<2>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+    } else {
+        direct_kernel<0>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+    }
     GI_HIP(hipGetLastError());
     if (timed) {
         GI_HIP(hipEventRecord(t0.b, st));
@@ -1477,7 +1494,7 @@ static NoAllocScratch* g_noalloc_ptr[64];  // per device, set once
 __global__ void k_noalloc_plan(NoAllocScratch* __restrict__ s, SimDesc sd, int nb, int ib) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) s->sim = sd;
-    if (b < nb) s->blocks[b] = DirectBlock{0, b * ib};
+    if (b < nb) s->blocks[b] = DirectBlock{0, b * ib, sd.start, sd.fe_end, sd.end, 0, 0, 0};
 }
 
 }  // namespace gi
@@ -1754,21 +1771,8 @@ int gi_force_collision_noalloc(const gi_float4* pos, const gi_float4* vel, gi_fl
     hipStream_t st = as_stream(stream);
     hipLaunchKernelGGL(k_noalloc_plan, dim3(nblk(nb, 256)), dim3(256), 0, st, sp, make_sim(0, c->NFe, n, law_of(c)),
                        nb, ib);
-    const dim3 grid(nb), block(64 * kDirectWaves);
-    const float4 *P = (const float4*)pos, *V = (const float4*)vel;
-    float4* F = (float4*)force;
-    if (lanes == 8)
-        hipLaunchKernelGGL((k_direct<false, 8, 0>), grid, block, 0, st, P, V, sp->blocks, &sp->sim, F, nullptr,
-                           FusedMove{});
-    else if (lanes == 4)
-        hipLaunchKernelGGL((k_direct<false, 4, 0>), grid, block, 0, st, P, V, sp->blocks, &sp->sim, F, nullptr,
-                           FusedMove{});
-    else if (lanes == 2)
-        hipLaunchKernelGGL((k_direct<false, 2, 0>), grid, block, 0, st, P, V, sp->blocks, &sp->sim, F, nullptr,
-                           FusedMove{});
-    else
-        hipLaunchKernelGGL((k_direct<false, 1, 0>), grid, block, 0, st, P, V, sp->blocks, &sp->sim, F, nullptr,
-                           FusedMove{});
+    direct_kernel<0>(lanes, direct_waves(n), nb, st, (const float4*)pos, (const float4*)vel, sp->blocks, &sp->sim,
+                     (float4*)force, FusedMove{});
     GI_HIP(hipGetLastError());
     return 0;
 }

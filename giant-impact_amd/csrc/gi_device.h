@@ -57,10 +57,11 @@ struct GroupTask {
     int kind, sim, group, j0, j1, piece, jfe, rtask0;
 };
 
-// One workgroup of the direct pass: 64 i-particles [i0, i0 + 64) of
-// simulation sim (the last block of a simulation may be ragged).
+// 64 / R i-particles from i0 on of simulation sim in the direct pass (the
+// last block of a simulation may be ragged), with the simulation's ranges
+// beside them: a workgroup starts from one load, not two in turn.
 struct DirectBlock {
-    int sim, i0;
+    int sim, i0, start, fe_end, end, pad0, pad1, pad2;
 };
 
 // The i-side slots of one row: slot0 .. slot0 + nslot - 1, in task order.

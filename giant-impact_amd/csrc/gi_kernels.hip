@@ -1102,27 +1102,29 @@ __global__ __launch_bounds__(64 * kContactWaves) void k_contact_corr(int ntot, c
 // ---------------------------------------------------------------------------
 //
 // For small N the three passes above are bound by their dozen launches, not by
-// arithmetic.  k_direct computes the same force in one: a workgroup holds
-// 64 / S i-particles, S lanes each, and its kDirectWaves * S lanes per
-// particle ("j-streams") share the simulation's j-range: each segment (iron
-// j, then silicate j, so the gravity product is one factor per segment) is
-// cut into groups of four j dealt out in turn (stream k takes groups k,
-// k + 16 S, ...).  Dealing keeps the contact work -- concentrated on the j
-// near the block's own particles -- spread over all streams; S > 1 gives small
-// simulations S times more wavefronts, each with a shorter chain (S = 8: 17%
-// faster steps at 2,048 particles than S = 4, whose workgroups fill only half
-// of the CUs there).  With S = 1
-// the j come through wave-uniform scalar loads.  Every pair takes the
-// all-pairs pass's branch-free gravity term (float tiles of kDirectTile j
-// folded into a compensated float sum); when some lane of a group has a pair
-// with r^2 < 1 the group also adds, for its pairs in contact, the exact
-// contact term minus that gravity term, with the arithmetic of k_finish.  The
-// streams' sums are added in a compensated float sum in a fixed order, so the
-// result depends on the simulation alone.  (The potential variant sums in
-// FP64: it feeds the energy reduction.)
-// POT: the per-particle potential of k_finish_potential instead of the force.
-constexpr int kDirectWaves = 16;
-constexpr int kDirectTile = 256;  // j per float tile
+// arithmetic.  k_direct computes the same force in one.  A workgroup holds
+// kDirectI i-particles, their positions wave-uniform (scalar registers); its
+// wavefronts deal out the simulation's 64-blocks of j, a j per lane, so that a
+// block's positions are one coalesced load for 64 kDirectI pairs and a step
+// is kDirectI independent chains.  (With the lanes over i and the j's
+// broadcast to them, each 64 pairs took a 16-byte load per lane: 16 cycles of
+// a CU's load path, which bounded the kernel: a step of N = 2,048, 4,096,
+// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 10.0, 15.2,
+// 32.0 and 53.)  It is bound by vector issue, 16 instructions per 64 pairs,
+// at the large end (11,000: 70% of the issue rate) and by the chain of loads,
+// step, contact terms and sums at the small end.  A wavefront's j are of one
+// material (the wavefronts are divided between the iron and the silicate j),
+// so the gravity product is one factor per wavefront and i.  Every pair takes
+// the all-pairs pass's branch-free gravity term into a float sum per lane and
+// i (N / 64 W terms for W wavefronts), added over the lanes as a tree.
+//
+// Pairs with r^2 < 1 are listed as they are met, in j order, one list per
+// wavefront; a full list and at the end what is left is worked off a pair per
+// lane: the exact contact term minus the gravity term, with the arithmetic of
+// k_finish, added per i in list order in a compensated sum.  The wavefronts'
+// sums are added in a compensated float sum in a fixed order, so the result
+// depends on the simulation and the number of wavefronts alone.
+constexpr int kDirectI = 8;
 // r^2 (with FMAs and kSelfEps) of every pair whose exactly rounded r is below
 // 1 lies below this: the margin covers the few ulps between the two forms.
 constexpr float kDirectContactR2 = 1.0001f;
@@ -1141,56 +1143,280 @@ struct FusedMove {
     float damp1, damp2;
 };
 
-// FP64 sum with CompSum's interface: the potential pass feeds the energy
-// reduction, which stays FP64.
-struct F64Sum {
-    double s;
-    __device__ __forceinline__ void zero() { s = 0.0; }
-    __device__ __forceinline__ void add(double x) { s += x; }
-    __device__ __forceinline__ double value() const { return s; }
-};
-struct PlainSum {
-    float s;
-    __device__ __forceinline__ void zero() { s = 0.0f; }
-    __device__ __forceinline__ void add(float x) { s += x; }
-    __device__ __forceinline__ float value() const { return s; }
-};
+template <int CTRL>
+__device__ __forceinline__ float lane_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+// lanes with `hi` keep y and send x to their partner, the others keep x
+template <int CTRL>
+__device__ __forceinline__ float lane_fold(float x, float y, bool hi) {
+    const float keep = hi ? y : x, send = hi ? x : y;
+    return keep + lane_dpp<CTRL>(send);
+}
+// x[k] summed over the 16 lanes of each row of lanes; lane p of the row gets
+// the sum of x[p & 7].
+__device__ __forceinline__ float row_sums8(const float (&x)[8], int p) {
+    float a[4], b[2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) a[k] = lane_fold<0x141>(x[k], x[k + 4], p & 4);  // lane p with 7 - p of its half row
+#pragma unroll
+    for (int k = 0; k < 2; ++k) b[k] = lane_fold<0x4E>(a[k], a[k + 2], p & 2);  // with p ^ 2
+    const float c = lane_fold<0xB1>(b[0], b[1], p & 1);                         // with p ^ 1
+    return c + lane_dpp<0x128>(c);                                              // with p ^ 8
+}
+// The four rows' x, y and z added: row 0 gets x, row 1 y, row 2 z.
+__device__ __forceinline__ float rows_sum_xyz(float x, float y, float z) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(z), false, false);
+    const float xz = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), 0u, false, false);
+    const float y0 = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+    const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(xz), __float_as_uint(y0), false, false);
+    return __uint_as_float(u[0]) + __uint_as_float(u[1]);
+}
 
-template <bool POT, int S, int MOVE>
-__global__ __launch_bounds__(64 * kDirectWaves) void k_direct(const float4* __restrict__ pos,
-                                                              const float4* __restrict__ vel,
-                                                              const DirectBlock* __restrict__ blocks,
-                                                              const SimDesc* __restrict__ sims,
-                                                              float4* __restrict__ force,
-                                                              double* __restrict__ pe, FusedMove mv) {
-    static_assert(MOVE == 0 || !POT, "the potential pass moves nothing");
+template <int MOVE, int W>
+__global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ pos,
+                                                   const float4* __restrict__ vel,
+                                                   const DirectBlock* __restrict__ blocks, int per_log2,
+                                                   const SimDesc* __restrict__ sims, float4* __restrict__ force,
+                                                   FusedMove mv) {
+    static_assert(W == 8 || W == 16, "wavefronts per workgroup");
+    constexpr int IB = kDirectI;
+    constexpr int kWorkOff = 128;             // listed pairs that are worked off before the next step
+    constexpr int kList = kWorkOff + 64 * IB;  // and what one step can add
+    __shared__ float grav[W][4 * 16];     // per wavefront: row c, lane p -> component c of i p
+    __shared__ float contact[W][6][IB];   // per wavefront: (sum, compensation) of x, y, z
+    __shared__ int list[W][kList];        // i << 24 | j
+    __shared__ float4 term[W][64];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const DirectBlock blk = blocks[blockIdx.x >> per_log2];
+    const int i0 = blk.i0 + IB * (blockIdx.x & ((1u << per_log2) - 1u));
+    const int start = blk.start, fe_end = blk.fe_end, end = blk.end;
+    const SimDesc& sd = sims[blk.sim];
+    if (i0 >= end) return;
+    float xi[IB], yi[IB], zi[IB];
+#pragma unroll
+    for (int k = 0; k < IB; ++k) {
+        const float4 p = pos[min(i0 + k, end - 1)];
+        xi[k] = p.x;
+        yi[k] = p.y;
+        zi[k] = p.z;
+    }
+    // the wavefronts that take iron j: their share of the 64-blocks
+    const int bf = (fe_end - start + 63) >> 6, bs = (end - fe_end + 63) >> 6;
+    const int wf = bf == 0 ? 0 : bs == 0 ? W : min(max((2 * W * bf + bf + bs) / (2 * (bf + bs)), 1), W - 1);
+    const bool jfe = wv < wf;
+    const int je = jfe ? fe_end : end;
+    const int stride = 64 * (jfe ? wf : W - wf);
+    int jb = jfe ? start + 64 * wv : fe_end + 64 * (wv - wf);  // the step's 64-block
+
+    float ax[IB], ay[IB], az[IB];
+#pragma unroll
+    for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
+    CompSum cx, cy, cz;  // lane k: the contact terms of i k
+    cx.zero();
+    cy.zero();
+    cz.zero();
+    int listed = 0;
+    const int steps = je <= jb ? 0 : (je - jb + stride - 1) / stride;
+    float4 nx = pos[min(jb + lane, end - 1)];
+    for (int st = 0;;) {
+        for (; st < steps && listed <= kWorkOff; ++st) {
+            float4 pj = nx;
+            const int j0 = jb;
+            jb += stride;
+            nx = pos[min(jb + lane, end - 1)];
+            if (j0 + lane >= je) pj.x = pj.y = pj.z = kGhostCoord;  // past the segment: no force, no contact
+            unsigned long long near[IB], any = 0;
+#pragma unroll
+            for (int k = 0; k < IB; ++k) {
+                const float dx = pj.x - xi[k];
+                const float dy = pj.y - yi[k];
+                const float dz = pj.z - zi[k];
+                const float r2 = fast_r2(dx, dy, dz);
+                const float s = fast_inv_r3(r2);
+                ax[k] = __builtin_fmaf(s, dx, ax[k]);
+                ay[k] = __builtin_fmaf(s, dy, ay[k]);
+                az[k] = __builtin_fmaf(s, dz, az[k]);
+                near[k] = __ballot(r2 < kDirectContactR2);
+                any |= near[k];
+            }
+            // the sums before the branch: sunk past it, their operands cost 32 registers
+#pragma unroll
+            for (int k = 0; k < IB; ++k) asm volatile("" : "+v"(ax[k]), "+v"(ay[k]), "+v"(az[k]));
+            if (!any) continue;
+#pragma unroll
+            for (int k = 0; k < IB; ++k) {
+                // not the pair of i k with itself, where this block holds it
+                const int own = i0 + k - j0;
+                unsigned long long m = near[k];
+                if (own >= 0 && own < 64 && i0 + k < je) m &= ~(1ull << own);
+                if (m == 0 || i0 + k >= end) continue;
+                if (m >> lane & 1)
+                    list[wv][listed + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+                        k << 24 | (j0 + lane);
+                listed += __popcll(m);
+            }
+        }
+        // The listed pairs: the exact contact term minus the gravity term
+        // s dp the sums took for it (k_finish's test and arithmetic), a pair
+        // per lane, then added per i in list order.
+                    // the law read here: hoisted out, its registers spill the loop's
+                    const SimDesc* lp = sims + blk.sim;
+                    asm volatile("" : "+s"(lp));
+                    const PairLaw& law = lp->law;
+                    for (int e0 = 0; e0 < listed; e0 += 64) {
+                        const int cnt = min(64, listed - e0);
+                        wave_lds_sync();
+                        float4 t = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
+                        if (lane < cnt) {
+                            const int e = list[wv][e0 + lane];
+                            const int k = e >> 24, jj = e & 0xffffff;
+                            const float4 pi = pos[i0 + k], pj = pos[jj];
+                            const float4 vi = vel[i0 + k], vj = vel[jj];
+                            const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+                            const float r2 = dx * dx + dy * dy + dz * dz;
+                            const float r = sqrtf(r2);
+                            if (r < 1.0f) {
+                                const float invr = 1.0f / r;
+                                const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+                                const float dot = dx * dvx + dy * dvy + dz * dvz;
+                                const int test = (int)(i0 + k < fe_end) + (int)jfe;
+                                const float fm = contact_pair_mag(law, test, r, r2, dot);
+                                const float sf = gravity_product(law, test) * fast_inv_r3(fast_r2(dx, dy, dz));
+                                t = make_float4(fm * dx * invr - sf * dx, fm * dy * invr - sf * dy, fm * dz * invr - sf * dz,
+                                                __int_as_float(k));
+                            }
+                        }
+                        term[wv][lane] = t;
+                        wave_lds_sync();
+                        // a batch's terms of one i: a handful, in a plain float sum
+                        float bx = 0.0f, by = 0.0f, bz = 0.0f;
+                        for (int q = 0; q < cnt; q += 4) {
+                            float4 u[4];
+        #pragma unroll
+                            for (int w = 0; w < 4; ++w) u[w] = term[wv][q + w];
+        #pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                const bool mine = __float_as_int(u[w].w) == lane;
+                                bx += mine ? u[w].x : 0.0f;
+                                by += mine ? u[w].y : 0.0f;
+                                bz += mine ? u[w].z : 0.0f;
+                            }
+                        }
+                        cx.add(bx);
+                        cy.add(by);
+                        cz.add(bz);
+                    }
+        if (st >= steps) break;
+        listed = 0;
+    }
+    grav[wv][lane] = rows_sum_xyz(row_sums8(ax, lane & 15), row_sums8(ay, lane & 15), row_sums8(az, lane & 15));
+    if (lane < IB) {
+        contact[wv][0][lane] = cx.s;
+        contact[wv][1][lane] = cx.c;
+        contact[wv][2][lane] = cy.s;
+        contact[wv][3][lane] = cy.c;
+        contact[wv][4][lane] = cz.s;
+        contact[wv][5][lane] = cz.c;
+    }
+    __syncthreads();
+    // Wavefront c < 3 adds component c: lane q * 8 + k takes the sums of i k
+    // of wavefronts q and q + 8, then the eight lanes of an i are added.  The
+    // move's components are independent; wavefront 3 carries .w over.
+    if (wv > 3) return;
+    const int k = lane & 7, q = lane >> 3;
+    const int i = i0 + k;
+    const bool ife = i < fe_end;
+    if (wv == 3) {
+        if constexpr (MOVE != 0)
+            if (lane < IB && i < end) {
+                mv.pout[i].w = pos[i].w;
+                mv.vout[i].w = vel[i].w;
+            }
+        return;
+    }
+    CompSum t;
+    t.zero();
+#pragma unroll
+    for (int u = 0; u < W / 8; ++u) {
+        const int w = q + 8 * u;
+        t.add_product(gravity_product(sd.law, (int)ife + (int)(w < wf)), grav[w][16 * wv + k]);
+        t.add(contact[w][2 * wv][k]);
+        t.c += contact[w][2 * wv + 1][k];
+    }
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) {
+        CompSum o;
+        o.s = __shfl_xor(t.s, m);
+        o.c = __shfl_xor(t.c, m);
+        t.add_sum(o);
+    }
+    if (lane >= IB || i >= end) return;
+    const float f = t.value();
+    reinterpret_cast<float*>(force + i)[wv] = f;
+    if constexpr (MOVE != 0) {
+        float temp, damp = 0.0f;
+        if constexpr (MOVE == 1) {
+            temp = i < mv.b1 ? mv.dt_over_mass_fe : mv.dt_over_mass_si;
+        } else if (mv.b3 <= i) {
+            temp = mv.dt_over_mass_si;
+            damp = mv.damp2;
+        } else if (mv.b2 <= i) {
+            temp = mv.dt_over_mass_fe;
+            damp = mv.damp2;
+        } else if (mv.b1 <= i) {
+            temp = mv.dt_over_mass_si;
+            damp = mv.damp1;
+        } else {
+            temp = mv.dt_over_mass_fe;
+            damp = mv.damp1;
+        }
+        float v = reinterpret_cast<const float*>(vel + i)[wv];
+        float p = reinterpret_cast<const float*>(pos + i)[wv];
+        if constexpr (MOVE == 1)
+            v += f * temp;
+        else
+            v += (f - damp * v) * temp;
+        p += v * mv.dt;
+        reinterpret_cast<float*>(mv.vout + i)[wv] = v;
+        reinterpret_cast<float*>(mv.pout + i)[wv] = p;
+    }
+}
+
+// The per-particle potential of k_finish_potential in one launch, for the
+// energy reduction (FP64 sums).  A workgroup holds 64 / S i-particles, S lanes
+// each, and its kDirectWaves * S lanes per particle ("j-streams") share the
+// simulation's j-range: each segment (iron j, then silicate j) is cut into
+// groups of four j dealt out in turn (stream k takes groups k, k + 16 S, ...),
+// summed in float tiles of kDirectTile j.
+constexpr int kDirectWaves = 16;
+constexpr int kDirectTile = 256;  // j per float tile
+
+template <int S>
+__global__ __launch_bounds__(64 * kDirectWaves) void k_direct_potential(const float4* __restrict__ pos,
+                                                                        const DirectBlock* __restrict__ blocks,
+                                                                        const SimDesc* __restrict__ sims,
+                                                                        double* __restrict__ pe) {
     static_assert(S == 1 || S == 2 || S == 4 || S == 8, "lanes per particle");
-    constexpr int IB = 64 / S;               // i-particles per workgroup
-    constexpr int NS = kDirectWaves * S;     // j-streams per particle
-    constexpr int TG = kDirectTile / 4;      // groups per stream per float tile
-    using Sum = typename std::conditional<POT, F64Sum, CompSum>::type;
-    using CSum = typename std::conditional<POT, F64Sum, PlainSum>::type;
-    using Val = typename std::conditional<POT, double, float>::type;
-    __shared__ Val red[3][kDirectWaves][64];
-    __shared__ float redc[POT ? 1 : 3][kDirectWaves][64];  // the force's compensations
+    constexpr int IB = 64 / S;             // i-particles per workgroup
+    constexpr int NS = kDirectWaves * S;   // j-streams per particle
+    constexpr int TG = kDirectTile / 4;    // groups per stream per float tile
+    __shared__ double red[kDirectWaves][64];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int stream = wv * S + lane / IB;  // wave-uniform when S == 1
     const DirectBlock b = blocks[blockIdx.x];
     const int start = sims[b.sim].start, fe_end = sims[b.sim].fe_end, end = sims[b.sim].end;
-    const PairLaw law = sims[b.sim].law;  // in registers: the contact branch reads it often
+    const PairLaw law = sims[b.sim].law;
     const int i = b.i0 + lane % IB;
     const bool live = i < end;
     const int ic = live ? i : end - 1;
     const float4 pi = pos[ic];
     const bool ife = ic < fe_end;
-
-    float4 vi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if constexpr (!POT) vi = vel[ic];
-    Sum sx, sy, sz;  // this wavefront's gravity plus contact corrections
-    sx.zero();
-    sy.zero();
-    sz.zero();
+    double sum = 0.0;  // this stream's gravity plus contact corrections
     for (int seg = 0; seg < 2; ++seg) {
         const bool jfe = seg == 0;  // iron j first, then silicate j
         const int a = jfe ? start : fe_end;
@@ -1199,216 +1425,69 @@ __global__ __launch_bounds__(64 * kDirectWaves) void k_direct(const float4* __re
         if (stream >= ngroups) continue;
         const int test = (int)ife + (int)jfe;
         const float g = gravity_product(law, test);
-        Sum ux, uy, uz;  // float tiles of kDirectTile j, folded (compensated; FP64 for the potential)
-        // this stream's contact terms of the segment: a handful (the pairs in
-        // contact are dealt over 16 S streams), so a plain float sum rounds
-        // them to ~3 ulp of their magnitudes; FP64 for the potential
-        CSum cx, cy, cz;
-        ux.zero();
-        uy.zero();
-        uz.zero();
-        cx.zero();
-        cy.zero();
-        cz.zero();
-        // The exact contact term of pair (i, j) minus the gravity term s*dp
-        // the tile sum took for it (k_finish's, resp. k_finish_potential's,
-        // test and arithmetic).
+        double u = 0.0, c = 0.0;
+        // k_finish_potential's term of a pair in contact
         auto contact = [&](int j, const float4 pj, float s) {
-            const float dx = pj.x - pi.x;
-            const float dy = pj.y - pi.y;
-            const float dz = pj.z - pi.z;
-            if constexpr (!POT) {
-                const float r2 = dx * dx + dy * dy + dz * dz;
-                if (!(r2 < 1.0f)) return;  // then sqrtf(r2) >= 1 too
-                const float r = sqrtf(r2);
-                if (r < 1.0f && j != i) {
-                    const float invr = 1.0f / r;
-                    const float4 vj = vel[j];
-                    const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
-                    const float dot = dx * dvx + dy * dvy + dz * dvz;
-                    const float fm = contact_pair_mag(law, test, r, r2, dot);
-                    const float sf = g * s;
-                    cx.add(fm * dx * invr - sf * dx);
-                    cy.add(fm * dy * invr - sf * dy);
-                    cz.add(fm * dz * invr - sf * dz);
-                }
-            } else {
-                const double ddx = (double)pj.x - pi.x, ddy = (double)pj.y - pi.y, ddz = (double)pj.z - pi.z;
-                const double r = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-                if (r < 1.0 && j != i) {
-                    const double G = gravity_product(law, test);
-                    const double K = approach_k(law, test);
-                    const double exact = G * (r - 2.0) + (K / 3.0) * (r - 1.0) * (r - 1.0) * (r + 2.0);
-                    cx.add(exact + G * (double)s);
-                }
+            const double ddx = (double)pj.x - pi.x, ddy = (double)pj.y - pi.y, ddz = (double)pj.z - pi.z;
+            const double r = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+            if (r < 1.0 && j != i) {
+                const double G = gravity_product(law, test);
+                const double K = approach_k(law, test);
+                const double exact = G * (r - 2.0) + (K / 3.0) * (r - 1.0) * (r - 1.0) * (r + 2.0);
+                c += exact + G * (double)s;
             }
         };
         // this stream's groups, TG of them per float tile
         for (int g0 = stream; g0 < ngroups; g0 += NS * TG) {
             const int g1 = min(g0 + NS * TG, ngroups);
-            float tx = 0.0f, ty = 0.0f, tz = 0.0f;
+            float tx = 0.0f;
             auto pair = [&](const float4 q, float& s, bool& near) {
                 const float dx = q.x - pi.x;
                 const float dy = q.y - pi.y;
                 const float dz = q.z - pi.z;
-                if constexpr (!POT) {
-                    const float r2f = fast_r2(dx, dy, dz);
-                    s = fast_inv_r3(r2f);
-                    tx = __builtin_fmaf(s, dx, tx);
-                    ty = __builtin_fmaf(s, dy, ty);
-                    tz = __builtin_fmaf(s, dz, tz);
-                    near |= r2f < kDirectContactR2;
-                } else {
-                    const float r2f = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-                    s = r2f > 0.0f ? __builtin_amdgcn_rsqf(r2f) : 0.0f;
-                    tx += s;
-                    near |= r2f < kDirectContactR2;
-                }
+                const float r2f = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                s = r2f > 0.0f ? __builtin_amdgcn_rsqf(r2f) : 0.0f;
+                tx += s;
+                near |= r2f < kDirectContactR2;
             };
             // The next group's loads are in flight while this one is computed
             // (indices clamped into the segment; a partial last group only
             // takes its first e - j pairs).
             float4 q[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = pos[min(a + 4 * g0 + u, e - 1)];
+            for (int k = 0; k < 4; ++k) q[k] = pos[min(a + 4 * g0 + k, e - 1)];
             for (int grp = g0; grp < g1; grp += NS) {
                 const int j = a + 4 * grp;
                 const int jn = grp + NS < g1 ? j + 4 * NS : j;
                 float4 nq[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) nq[u] = pos[min(jn + u, e - 1)];
+                for (int k = 0; k < 4; ++k) nq[k] = pos[min(jn + k, e - 1)];
                 float s[4];
                 bool near = false;
-                if (j + 4 <= e) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) pair(q[u], s[u], near);
-                    if (near) {
+                for (int k = 0; k < 4; ++k)
+                    if (j + k < e) pair(q[k], s[k], near);
+                if (near) {
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) contact(j + u, q[u], s[u]);
-                    }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (j + u < e) pair(q[u], s[u], near);
-                    if (near) {
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (j + u < e) contact(j + u, q[u], s[u]);
-                    }
+                    for (int k = 0; k < 4; ++k)
+                        if (j + k < e) contact(j + k, q[k], s[k]);
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) q[u] = nq[u];
+                for (int k = 0; k < 4; ++k) q[k] = nq[k];
             }
-            ux.add(tx);
-            uy.add(ty);
-            uz.add(tz);
+            u += (double)tx;
         }
-        if constexpr (!POT) {
-            sx.add_product(g, ux.s);
-            sx.c += g * ux.c;
-            sx.add(cx.s);
-            sy.add_product(g, uy.s);
-            sy.c += g * uy.c;
-            sy.add(cy.s);
-            sz.add_product(g, uz.s);
-            sz.c += g * uz.c;
-            sz.add(cz.s);
-        } else {
-            sx.add(-(double)g * ux.value() + cx.value());
-        }
+        sum += -(double)g * u + c;
     }
-    if constexpr (!POT) {
-        red[0][wv][lane] = sx.s;
-        red[1][wv][lane] = sy.s;
-        red[2][wv][lane] = sz.s;
-        redc[0][wv][lane] = sx.c;
-        redc[1][wv][lane] = sy.c;
-        redc[2][wv][lane] = sz.c;
-    } else {
-        red[0][wv][lane] = sx.value();
-    }
+    red[wv][lane] = sum;
     __syncthreads();
-    // The force: wavefronts 0-2 take one component each; lane (q, p) adds the
-    // 16 wavefronts' partials of particle p's q-th stream in wavefront order,
-    // then the S streams' sums are added in order (a 16 + S chain per lane
-    // instead of a 16 S chain on one wavefront).  The potential: one FP64
-    // chain on wavefront 0.
-    __shared__ float part[POT ? 1 : 3][2][64];
-    if constexpr (!POT) {
-        if (wv < 3) {
-            CompSum a;
-            a.zero();
-#pragma unroll
-            for (int w = 0; w < kDirectWaves; ++w) {
-                a.add(red[wv][w][lane]);
-                a.c += redc[wv][w][lane];
-            }
-            part[wv][0][lane] = a.s;
-            part[wv][1][lane] = a.c;
-        }
-        __syncthreads();
-    }
     if (wv == 0 && lane < IB && live) {
-        if constexpr (!POT) {
-            float f[3];
+        double f = 0.0;
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                CompSum t;
-                t.zero();
+        for (int w = 0; w < kDirectWaves; ++w)
 #pragma unroll
-                for (int q = 0; q < S; ++q) {
-                    t.add(part[c][0][q * IB + lane]);
-                    t.c += part[c][1][q * IB + lane];
-                }
-                f[c] = t.value();
-            }
-            const float f0 = f[0], f1 = f[1], f2 = f[2];
-            force[i].x = f0;
-            force[i].y = f1;
-            force[i].z = f2;
-            if constexpr (MOVE != 0) {
-                float temp, damp = 0.0f;
-                if constexpr (MOVE == 1) {
-                    temp = i < mv.b1 ? mv.dt_over_mass_fe : mv.dt_over_mass_si;
-                } else if (mv.b3 <= i) {
-                    temp = mv.dt_over_mass_si;
-                    damp = mv.damp2;
-                } else if (mv.b2 <= i) {
-                    temp = mv.dt_over_mass_fe;
-                    damp = mv.damp2;
-                } else if (mv.b1 <= i) {
-                    temp = mv.dt_over_mass_si;
-                    damp = mv.damp1;
-                } else {
-                    temp = mv.dt_over_mass_fe;
-                    damp = mv.damp1;
-                }
-                float4 v = vel[i];
-                float4 p = pos[i];
-                if constexpr (MOVE == 1) {
-                    v.x += f0 * temp;
-                    v.y += f1 * temp;
-                    v.z += f2 * temp;
-                } else {
-                    v.x += (f0 - damp * v.x) * temp;
-                    v.y += (f1 - damp * v.y) * temp;
-                    v.z += (f2 - damp * v.z) * temp;
-                }
-                p.x += v.x * mv.dt;
-                p.y += v.y * mv.dt;
-                p.z += v.z * mv.dt;
-                mv.vout[i] = v;
-                mv.pout[i] = p;
-            }
-        } else {
-            F64Sum fx;
-            fx.zero();
-#pragma unroll
-            for (int w = 0; w < kDirectWaves; ++w)
-#pragma unroll
-                for (int q = 0; q < S; ++q) fx.add(red[0][w][q * IB + lane]);
-            pe[i] = 0.5 * fx.value();
-        }
+            for (int q = 0; q < S; ++q) f += red[w][q * IB + lane];
+        pe[i] = 0.5 * f;
     }
 }
 
@@ -2084,18 +2163,23 @@ GI_GRAVITY_INST(8, true, 0)
 #undef GI_GRAVITY_INST
 #define GI_MUTUAL_INST(R, POT) \
     template __global__ void k_mutual<R, POT>(const float4*, const MutualTask*, int, const SimDesc*, float*, float*);
-#define GI_DIRECT_INST(POT, S, MOVE)                                                                 \
-    template __global__ void k_direct<POT, S, MOVE>(const float4*, const float4*, const DirectBlock*, \
-                                                    const SimDesc*, float4*, double*, FusedMove);
-#define GI_DIRECT_INST_S(S)       \
-    GI_DIRECT_INST(false, S, 0)   \
-    GI_DIRECT_INST(false, S, 1)   \
-    GI_DIRECT_INST(false, S, 2)   \
-    GI_DIRECT_INST(true, S, 0)
-GI_DIRECT_INST_S(1)
-GI_DIRECT_INST_S(2)
-GI_DIRECT_INST_S(4)
-GI_DIRECT_INST_S(8)
+#define GI_DIRECT_INST(MOVE, W)                                                                            \
+    template __global__ void k_direct<MOVE, W>(const float4*, const float4*, const DirectBlock*, int,      \
+                                               const SimDesc*, float4*, FusedMove);
+GI_DIRECT_INST(0, 8)
+GI_DIRECT_INST(1, 8)
+GI_DIRECT_INST(2, 8)
+GI_DIRECT_INST(0, 16)
+GI_DIRECT_INST(1, 16)
+GI_DIRECT_INST(2, 16)
+#undef GI_DIRECT_INST
+#define GI_DIRECT_POT_INST(S) \
+    template __global__ void k_direct_potential<S>(const float4*, const DirectBlock*, const SimDesc*, double*);
+GI_DIRECT_POT_INST(1)
+GI_DIRECT_POT_INST(2)
+GI_DIRECT_POT_INST(4)
+GI_DIRECT_POT_INST(8)
+#undef GI_DIRECT_POT_INST
 GI_MUTUAL_INST(1, false)
 GI_MUTUAL_INST(2, false)
 GI_MUTUAL_INST(4, false)

@@ -178,7 +178,7 @@ int gi_force_collision(const gi_float4 *pos, const gi_float4 *vel, gi_float4 *fo
  * loops, harnesses that forbid hipMalloc): the same force, bitwise, where the
  * tuning table gives gi_force_collision the direct pass (n <= 12,288), with
  * the direct pass's scratch (the simulation descriptor and the block table,
- * ~13 KB) in a static device array that each device holds until the process
+ * ~50 KB) in a static device array that each device holds until the process
  * ends.  Allocates nothing, host or device.  n > 12,288 returns
  * GI_E_TOO_LARGE.  Every call on one device shares that array: calls that
  * overlap on one device (several host threads, or several streams without
