@@ -140,7 +140,8 @@ struct Workspace {
     DevBuf<RowDesc> rows;
     DevBuf<SumBlock> sblocks;
     DevBuf<DirectBlock> dblocks;
-    DevBuf<int> counts, starts, sorted, cellhash, block_sums;
+    DevBuf<int> counts, lstarts, starts, slots, sorted, block_sums;
+    DevBuf<int2> place;  // each particle's bucket and place of arrival in it
     DevBuf<float4> spos, svel;  // positions / velocities in bucket order
     DevBuf<float> corr;         // contact corrections: per particle (sum, compensation) of x, y, z
     DevBuf<GravTask> tasks;
@@ -795,6 +796,8 @@ static int check_plan_indexes(const Plan& p) {
     return 0;
 }
 
+static inline int nblk(long long n, int b) { return (int)((n + b - 1) / b); }
+
 template <typename T>
 static int upload(DevBuf<T>& b, const std::vector<T>& v, hipStream_t st) {
     int rc = b.ensure(v.size());
@@ -836,11 +839,15 @@ static int ensure_plan(Workspace* ws, const std::vector<SimDesc>& sims, hipStrea
     }
     if (p.direct && (rc = upload(ws->dblocks, p.dblocks, st))) return rc;
     if ((rc = ws->counts.ensure((size_t)p.buckets + 1))) return rc;
+    hipLaunchKernelGGL(k_fill_int, dim3(nblk(p.buckets, 256)), dim3(256), 0, st, ws->counts.p, p.buckets, 0);
+    GI_HIP(hipGetLastError());
+    if ((rc = ws->lstarts.ensure((size_t)p.buckets + 1))) return rc;
     if ((rc = ws->starts.ensure((size_t)p.buckets + 2))) return rc;
+    if ((rc = ws->slots.ensure((size_t)p.ntot + 1))) return rc;
+    if ((rc = ws->place.ensure((size_t)p.ntot + 1))) return rc;
     if ((rc = ws->spos.ensure((size_t)p.ntot + 1))) return rc;
     if ((rc = ws->svel.ensure((size_t)p.ntot + 1))) return rc;
     if ((rc = ws->sorted.ensure((size_t)p.ntot + 1))) return rc;
-    if ((rc = ws->cellhash.ensure((size_t)p.ntot + 1))) return rc;
     if ((rc = ws->block_sums.ensure((size_t)p.buckets / 1024 + 8))) return rc;
     if ((rc = upload(ws->tasks, p.tasks, st))) return rc;
     if ((rc = upload(ws->sims, p.sims, st))) return rc;
@@ -857,33 +864,27 @@ static int ensure_plan(Workspace* ws, const std::vector<SimDesc>& sims, hipStrea
     return 0;
 }
 
-static inline int nblk(long long n, int b) { return (int)((n + b - 1) / b); }
-
 // ---------------------------------------------------------------------------
 // Launch sequences
 // ---------------------------------------------------------------------------
 
-// Contact grid of the current plan: bucket counts, offsets (scan), particle
-// ids per bucket sorted by id, and positions / velocities in that order
-// (vel may be null when only positions are needed).
+// Contact grid of the current plan: bucket offsets, particle ids per bucket
+// sorted by id, and positions / velocities in that order (vel may be null
+// when only positions are needed).  The counts are zero before and after.
 static int launch_grid(Workspace* ws, const float4* pos, const float4* vel, hipStream_t st) {
     const Plan& p = ws->plan;
     const int m = p.buckets;
     const int nsims = (int)p.sims.size();
-    hipLaunchKernelGGL(k_fill_int, dim3(nblk(m, 256)), dim3(256), 0, st, ws->counts.p, m, 0);
     hipLaunchKernelGGL(k_grid_count, dim3(nblk(p.ntot, 256)), dim3(256), 0, st, pos, p.ntot, ws->sims.p,
-                       nsims, ws->counts.p, ws->cellhash.p);
+                       nsims, ws->counts.p, ws->place.p);
     const int nb = nblk(m, 1024);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, st, ws->counts.p, m, ws->starts.p,
+    hipLaunchKernelGGL(k_scan_blocks<true>, dim3(nb), dim3(256), 0, st, ws->counts.p, m, ws->lstarts.p,
                        ws->block_sums.p);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, st, ws->block_sums.p, nb, ws->starts.p + m);
-    hipLaunchKernelGGL(k_scan_add, dim3(nblk(m, 256)), dim3(256), 0, st, ws->starts.p, m, ws->block_sums.p);
-    hipLaunchKernelGGL(k_grid_scatter, dim3(nblk(p.ntot, 256)), dim3(256), 0, st, p.ntot, ws->cellhash.p,
-                       ws->starts.p, ws->counts.p, ws->sorted.p);
-    hipLaunchKernelGGL(k_grid_sort_buckets, dim3(nblk(m, 256)), dim3(256), 0, st, m, ws->starts.p,
-                       ws->sorted.p);
-    hipLaunchKernelGGL(k_grid_gather, dim3(nblk(p.ntot, 256)), dim3(256), 0, st, p.ntot,
-                       (const int*)ws->sorted.p, pos, vel, ws->spos.p, vel ? ws->svel.p : nullptr);
+    hipLaunchKernelGGL(k_grid_place, dim3(nblk(std::max(m, p.ntot), 256)), dim3(256), 0, st, p.ntot, m,
+                       ws->lstarts.p, ws->block_sums.p, ws->place.p, ws->starts.p, ws->slots.p);
+    hipLaunchKernelGGL(k_grid_rank, dim3(nblk(p.ntot, 256)), dim3(256), 0, st, p.ntot, ws->slots.p, ws->place.p,
+                       ws->starts.p, pos, vel, ws->sorted.p, ws->spos.p, vel ? ws->svel.p : nullptr);
     GI_HIP(hipGetLastError());
     return 0;
 }
@@ -1912,7 +1913,7 @@ int gi_find_earth_moon(const gi_float4* pos, const gi_float4* vel, int n, int nf
     hipLaunchKernelGGL(k_fill_int, dim3(nblk(m, 256)), dim3(256), 0, st, w.counts.p, (int)m, 0);
     hipLaunchKernelGGL(k_cc_count, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, inv_c, m - 1, w.counts.p,
                        w.cellhash.p, w.size.p);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nbs), dim3(256), 0, st, w.counts.p, (int)m, w.starts.p, w.block_sums.p);
+    hipLaunchKernelGGL(k_scan_blocks<false>, dim3(nbs), dim3(256), 0, st, w.counts.p, (int)m, w.starts.p, w.block_sums.p);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, st, w.block_sums.p, nbs, w.starts.p + m);
     hipLaunchKernelGGL(k_scan_add, dim3(nblk(m, 256)), dim3(256), 0, st, w.starts.p, (int)m, w.block_sums.p);
     hipLaunchKernelGGL(k_cc_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, w.cellhash.p, w.starts.p, w.counts.p,

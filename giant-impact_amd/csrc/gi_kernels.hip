@@ -759,20 +759,30 @@ __global__ void k_fill_int(int* __restrict__ a, int n, int v) {
     if (i < n) a[i] = v;
 }
 
+// The grid takes five launches (it can be the critical path beside the pair
+// kernel of a mid-size plan, where each launch of a chain is 5 us): the
+// buckets' counts with each particle's place of arrival in its bucket; the
+// scan of every 1,024 counts, which leaves them at zero for the next grid;
+// the scan of the block totals; the particles at their places; and each
+// particle at its rank by id among its bucket's, with its position and
+// velocity.  (Cleared, counted, scanned in three launches, scattered, sorted
+// a bucket per lane and gathered took eight; the block totals summed by every
+// workgroup of k_grid_place for itself took its 256 lanes and their barriers
+// 50 us beside a running pair kernel.)
 __global__ void k_grid_count(const float4* __restrict__ pos, int ntot, const SimDesc* __restrict__ sims,
-                             int nsims, int* __restrict__ counts, int* __restrict__ cellhash) {
+                             int nsims, int* __restrict__ counts, int2* __restrict__ place) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ntot) return;
     const SimDesc& sd = sims[find_sim(sims, nsims, i)];
     float4 p = pos[i];
     unsigned h = cell_bucket(sd.hbase, sd.hmask, cell_coord(p.x), cell_coord(p.y), cell_coord(p.z));
-    cellhash[i] = (int)h;
-    atomicAdd(&counts[h], 1);
+    place[i] = make_int2((int)h, atomicAdd(&counts[h], 1));
 }
 
-// Exclusive scan of counts[0..m) into starts[0..m], 1024 elements per block.
-__global__ __launch_bounds__(256) void k_scan_blocks(const int* __restrict__ in, int m,
-                                                     int* __restrict__ out,
+// Exclusive scan of in[0..m) into out[0..m], 1024 elements per block; CLEAR
+// leaves in[] at zero.
+template <bool CLEAR>
+__global__ __launch_bounds__(256) void k_scan_blocks(int* __restrict__ in, int m, int* __restrict__ out,
                                                      int* __restrict__ block_sums) {
     __shared__ int sh[256];
     const int base = blockIdx.x * 1024 + threadIdx.x * 4;
@@ -781,6 +791,7 @@ __global__ __launch_bounds__(256) void k_scan_blocks(const int* __restrict__ in,
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         v[k] = (base + k < m) ? in[base + k] : 0;
+        if (CLEAR && base + k < m) in[base + k] = 0;
         local += v[k];
     }
     sh[threadIdx.x] = local;
@@ -840,43 +851,36 @@ __global__ void k_scan_add(int* __restrict__ out, int m, const int* __restrict__
     if (i < m) out[i] += block_sums[i >> 10];
 }
 
-// Scatter particle ids into their buckets; counts[] is consumed back to zero.
-__global__ void k_grid_scatter(int ntot, const int* __restrict__ cellhash,
-                               const int* __restrict__ starts, int* __restrict__ counts,
-                               int* __restrict__ sorted) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ntot) return;
-    int h = cellhash[i];
-    int slot = starts[h] + atomicSub(&counts[h], 1) - 1;
-    sorted[slot] = i;
-}
-
-// Sort each bucket by particle id so the contact sums run in a fixed order.
-__global__ void k_grid_sort_buckets(int m, const int* __restrict__ starts, int* __restrict__ sorted) {
-    int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= m) return;
-    int s = starts[h], e = starts[h + 1];
-    for (int a = s + 1; a < e; ++a) {
-        int key = sorted[a];
-        int b = a - 1;
-        while (b >= s && sorted[b] > key) {
-            sorted[b + 1] = sorted[b];
-            --b;
-        }
-        sorted[b + 1] = key;
+// The bucket offsets of the whole grid (starts[0..m)) and the particle ids at
+// their places of arrival (slots), from the scan's blocks (lstarts,
+// block_sums): buckets and particles are dealt out over one grid.
+__global__ void k_grid_place(int ntot, int m, const int* __restrict__ lstarts, const int* __restrict__ block_sums,
+                             const int2* __restrict__ place, int* __restrict__ starts, int* __restrict__ slots) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < m) starts[t] = lstarts[t] + block_sums[t >> 10];
+    if (t < ntot) {
+        const int2 p = place[t];
+        slots[lstarts[p.x] + block_sums[p.x >> 10] + p.y] = t;
     }
 }
 
-// Positions and velocities in bucket order, so the contact pass reads the
-// particles of a cell from consecutive memory.
-__global__ void k_grid_gather(int ntot, const int* __restrict__ sorted, const float4* __restrict__ pos,
-                              const float4* __restrict__ vel, float4* __restrict__ spos,
-                              float4* __restrict__ svel) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+// Each particle at its rank by id among its bucket's particles, so that the
+// contact sums run in a fixed order, with its position and velocity: the
+// contact pass reads the particles of a cell from consecutive memory.
+__global__ void k_grid_rank(int ntot, const int* __restrict__ slots, const int2* __restrict__ place,
+                            const int* __restrict__ starts, const float4* __restrict__ pos,
+                            const float4* __restrict__ vel, int* __restrict__ sorted, float4* __restrict__ spos,
+                            float4* __restrict__ svel) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntot) return;
-    const int i = sorted[t];
-    spos[t] = pos[i];
-    if (svel) svel[t] = vel[i];
+    const int i = slots[t];
+    const int h = place[i].x;
+    const int s = starts[h], e = starts[h + 1];
+    int at = s;
+    for (int k = s; k < e; ++k) at += slots[k] < i;
+    sorted[at] = i;
+    spos[at] = pos[i];
+    if (svel) svel[at] = vel[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -898,7 +902,11 @@ __global__ void k_grid_gather(int ntot, const int* __restrict__ sorted, const fl
 // particles per wavefront, the row sums added through LDS): a chain a ninth
 // as long, for plans too small to hide the walk behind the all-pairs pass.
 // LANES = 1 walks them in turn on one lane.  The arithmetic is the same, so
-// the two forms give bitwise the same corrections.  A simulation's buckets
+// the two forms give bitwise the same corrections.  No candidate's cell is
+// looked at: a bucket may hold particles of other cells, but the 27 cells
+// have 27 buckets (a simulation has at least 4 x 4 x 4), a pair with r < 1
+// lies in adjacent cells (coordinates a unit apart or more round to a
+// difference of one or more), and so it is met in one bucket alone.  A simulation's buckets
 // hold only its own particles, and the particle itself sits at position t,
 // so a candidate's index is loaded only for a pair in contact.
 constexpr int kCellRows = 9;
@@ -922,11 +930,9 @@ __device__ __forceinline__ void contact_row(const SimDesc& sd, int t, int i, int
     }
 #pragma unroll
     for (int ox = 0; ox < 3; ++ox) {
-        const int qx = ccx + ox - 1;
         for (int k = b0[ox]; k < b1[ox]; ++k) {
             const float4 pj = spos[k];
-            if (k == t || cell_coord(pj.x) != qx || cell_coord(pj.y) != qy || cell_coord(pj.z) != qz)
-                continue;  // i itself, or another cell sharing the bucket
+            if (k == t) continue;  // i itself
             const float dpx = pj.x - pi.x;
             const float dpy = pj.y - pi.y;
             const float dpz = pj.z - pi.z;
