@@ -286,7 +286,7 @@ constexpr long long kMutualMaxChunk = 4096;
 // work of a piece of L.  A row's i-side slots are its group's pieces in
 // order, then its diagonal pieces, then its in-group tasks: contiguous, as
 // the sums expect.  In the batched engine each simulation's L is the
-// engine's, shortened to N / kBatchedPieceDiv (whole 64-blocks, at least
+// engine's, shortened to N / batched_piece_div(N) (whole 64-blocks, at least
 // one) for simulations too small to fill the GPU with pieces of the full
 // length: a function of the simulation alone, so its sums are the same in
 // any batch.  In a single-simulation plan the last groups (the shortest
@@ -300,7 +300,14 @@ constexpr long long kMutualMaxChunk = 4096;
 // L / 2 (one 30,000-particle simulation stepped 16% faster, eight mixed ones
 // 2%, the 64-simulation ensemble the same within 0.2%; a quarter and a
 // sixteenth gained less).
-constexpr long long kBatchedPieceDiv = 32;
+//
+// The divisor: a small company's step lasts as long as its longest tasks, a
+// large one's is the longer the more slots there are.  At 32 throughout,
+// eight simulations of 4,000 to 18,600 particles step in 0.279 ms, four of
+// 12,300 to 18,000 in 0.312; as below 0.238 and 0.258, and the 64-simulation
+// ensemble the same (4.64 ms; 1.1% slower at 64 throughout).  One of 30,000
+// is 2% faster at 32 than at 48.
+static long long batched_piece_div(long long n) { return n <= 12288 ? 64 : n <= 24576 ? 48 : 32; }
 constexpr long long kTailPieces = 1536;
 constexpr long long kBatchedTailDiv = 8;
 
@@ -310,8 +317,8 @@ static int plan_mutual_groups(const std::vector<SimDesc>& sims, const Tiling& tl
     for (size_t si = 0; si < sims.size(); ++si) {
         const SimDesc& s = sims[si];
         if (s.gn == 0) continue;
-        const long long L = batched ? std::min(L0, std::max(64LL, ((s.end - s.start) / kBatchedPieceDiv + 63) / 64 * 64))
-                                    : L0;
+        const long long n = s.end - s.start;
+        const long long L = batched ? std::min(L0, std::max(64LL, (n / batched_piece_div(n) + 63) / 64 * 64)) : L0;
         const int nrows = s.gn / B;
         const int fe_real = (s.fe_end - s.start + 63) / 64 * 64;
         const int si_real = s.gfe + (s.end - s.fe_end + 63) / 64 * 64;
@@ -542,9 +549,12 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
 static std::atomic<int> g_contact_overlap{1};  // see gi_set_contact_overlap
 static std::atomic<int> g_contact_walk{0};     // see gi_set_contact_walk
 
-// The contact walk for plans of up to this many particles uses nine lanes per
-// particle: their all-pairs pass is too short to hide a one-lane walk.
-constexpr int kContactRowLanesMaxN = 49152;
+// The contact walk of plans of up to this many pairs (a simulation of 49,152
+// particles, or several smaller ones) uses nine lanes per particle: their
+// all-pairs pass, up to 0.4 ms, is too short to hide a one-lane walk of 0.2
+// to 0.4 ms and the grid before it (eight simulations of 77,000 particles
+// together, a pass of 0.26 ms: 0.275 ms a step with nine lanes, 0.285 with one).
+constexpr double kContactRowLanesMaxPairs = 49152.0 * 49152.0;
 
 static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched, Plan* out) {
     Plan p;
@@ -644,7 +654,10 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
     }
     p.overlap_allowed = g_contact_overlap.load() != 0;
     p.contact_walk = g_contact_walk.load();
-    p.contact_lanes = p.contact_walk ? p.contact_walk : (p.ntot <= kContactRowLanesMaxN ? 9 : 1);
+    double pairs = 0.0;
+    for (const SimDesc& s : sims)
+        if (s.active) pairs += (double)(s.end - s.start) * (double)(s.end - s.start);
+    p.contact_lanes = p.contact_walk ? p.contact_walk : (pairs <= kContactRowLanesMaxPairs ? kCellRows : 1);
     p.split_finish = p.mutual && p.tasks.empty() && !p.direct && p.overlap_allowed;
     p.sims = std::move(sims);
     *out = std::move(p);
