@@ -412,6 +412,31 @@ static long long group_slab_entries(long long gn, long long nrows, int B, int W)
     return e;
 }
 
+// The 64 places from q0 on of simulation s (number si) as a workgroup of
+// k_mutual_sum, with rows of B places in groups of W.
+static SumBlock sum_block(const SimDesc& s, int si, int q0, int B, int W, const RowDesc& rd) {
+    const bool iron = q0 < s.gfe;
+    const int row = q0 / B, group = row / W;
+    const int i0 = iron ? s.start + q0 : s.fe_end + (q0 - s.gfe);
+    SumBlock b{};
+    b.sim = si;
+    b.q0 = q0;
+    b.i0 = i0;
+    b.nreal = std::min(64, (iron ? s.fe_end : s.end) - i0);
+    b.slot0 = rd.slot0;
+    b.nslot = rd.nslot;
+    b.group = group;
+    b.in_group = row - group * W;
+    // entry q - (g + 1) W B of group g's slab; entry q - (r + 1) B of row
+    // r's (W - 1) B entries in its group
+    const long long first = (long long)group * W, ilen = (long long)(W - 1) * B;
+    b.jfirst = s.jbase + 3 * (q0 - (long long)W * B);
+    b.ifirst = s.jibase + 3 * (ilen * first + q0 - (first + 1) * B);
+    b.gn = s.gn;
+    b.iron = iron;
+    return b;
+}
+
 static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batched, Plan& p) {
     const int B = 64 * tl.R;
     const int W = tl.variant == 4 ? kGroupRows : 1;
@@ -498,9 +523,8 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
         const int nfe = s.fe_end - s.start, nsi = s.end - s.fe_end;
         for (int q0 = 0; q0 < s.gn; q0 += 64) {
             if (q0 < s.gfe ? q0 >= nfe : q0 - s.gfe >= nsi) continue;  // ghosts only
-            const int I = q0 / B;
-            sblocks.push_back(SumBlock{(int)si, q0});
-            swork.push_back(rows[s.row0 + I].nslot + I / W + I % W);
+            sblocks.push_back(sum_block(s, (int)si, q0, B, W, rows[s.row0 + q0 / B]));
+            swork.push_back(sblocks.back().nslot + sblocks.back().group + sblocks.back().in_group);
         }
     }
     std::vector<int> order(sblocks.size());
@@ -757,20 +781,33 @@ static int check_plan_indexes(const Plan& p) {
     for (const SumBlock& b : p.sblocks) {
         GI_CHECK(b.sim >= 0 && b.sim < (int)p.sims.size(), "sum block sim");
         const SimDesc& sd = p.sims[b.sim];
-        GI_CHECK(b.q0 % 64 == 0 && b.q0 + 64 <= sd.gn, "sum block places");
+        GI_CHECK(b.q0 >= 0 && b.q0 % 64 == 0 && b.q0 + 64 <= sd.gn, "sum block places");
         const int row = b.q0 / B, group = row / W;
         const long long WB = (long long)W * B, ilen = (long long)(W - 1) * B;
+        const RowDesc& rd = p.rows[sd.row0 + row];
+        GI_CHECK(b.slot0 == rd.slot0 && b.nslot == rd.nslot && b.group == group && b.in_group == row - group * W &&
+                     b.gn == sd.gn && (b.iron != 0) == (b.q0 < sd.gfe),
+                 "sum block lists");
+        GI_CHECK(b.iron ? b.i0 == sd.start + b.q0 && b.i0 + b.nreal <= sd.fe_end
+                        : b.i0 == sd.fe_end + (b.q0 - sd.gfe) && b.i0 + b.nreal <= sd.end,
+                 "sum block particles");
+        GI_CHECK(b.nreal > 0 && b.nreal <= 64, "sum block size");
         for (int q = b.q0; q < b.q0 + 64; ++q) {
             for (int g = 0; g < group; ++g) {
                 const long long len = sd.gn - (g + 1) * WB;
                 const long long o = q - (g + 1) * WB;
                 GI_CHECK(o >= 0 && o < len, "sum: group entry");
                 GI_CHECK(sd.jbase + 3 * (jside_row_offset(g, sd.gn, WB) + o) + 2 < p.jside_len, "sum: J");
+                GI_CHECK(b.jfirst + 3 * sum_group_offset(g, sd.gn, WB) + 3 * (q - b.q0) ==
+                             sd.jbase + 3 * (jside_row_offset(g, sd.gn, WB) + o),
+                         "sum: group entry's place");
             }
             for (int r2 = group * W; r2 < row; ++r2) {
                 const long long o = q - (long long)(r2 + 1) * B;
                 GI_CHECK(o >= 0 && o < ilen && sd.jibase + 3 * (ilen * r2 + o) + 2 < p.jintra_len,
                          "sum: in-group entry");
+                GI_CHECK(b.ifirst + 3 * (ilen - B) * (r2 - group * W) + 3 * (q - b.q0) == sd.jibase + 3 * (ilen * r2 + o),
+                         "sum: in-group entry's place");
             }
         }
     }
@@ -971,6 +1008,13 @@ static void launch_mutual_kernel(int R, hipStream_t st, const Workspace* ws, int
                            ws->iside.p, ws->jside.p);
 }
 
+// Steps enqueued together (a multi-step graph) whose move is fused into
+// k_mutual_sum: the padded copy of a step's positions is left by the step
+// before it (kCarryOut there, kCarryIn here) instead of made by k_mutual_pad.
+// Nothing else writes the positions or the copy between the two.
+enum PadCarry { kCarryIn = 1, kCarryOut = 2 };
+static int pad_carry(int step, int steps) { return (step > 0 ? kCarryIn : 0) | (step + 1 < steps ? kCarryOut : 0); }
+
 // The all-pairs pass of the current plan: the one-sided kernel for the
 // simulations planned one-sided, and for the others the mutual pass (padded
 // copy, pair kernel, per-particle sums into ws->gsum).  Timed: kind 0 spans
@@ -985,7 +1029,7 @@ static void launch_mutual_kernel(int R, hipStream_t st, const Workspace* ws, int
 static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool pot, hipStream_t st,
                           bool timed, float4* force = nullptr, hipEvent_t join = nullptr, hipEvent_t fork = nullptr,
                           const std::function<int()>& side_work = nullptr, float4* mpos = nullptr,
-                          float4* mvel = nullptr, const SumMove& mv = SumMove{0.0f, 0.0f, 0.0f, 1}) {
+                          float4* mvel = nullptr, const SumMove& mv = SumMove{}, int carry = 0) {
     const Plan& p = ws->plan;
     const int nplain = (int)p.tasks.size();
     const bool grouped = p.group_rows > 1;
@@ -1003,7 +1047,7 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
         pass = take_pair(ctx, 2);
         GI_HIP(hipEventRecord(pass.a, st));
     }
-    if (nmut > 0)
+    if (nmut > 0 && !(carry & kCarryIn))
         hipLaunchKernelGGL(k_mutual_pad, dim3(nblk(p.gtot, 256)), dim3(256), 0, st, pos, (int)p.gtot, ws->sims.p,
                            nsims, ws->gpos.p);
     if (fork) GI_HIP(hipEventRecord(fork, st));
@@ -1046,14 +1090,15 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
     if (nmut > 0 && !p.sblocks.empty()) {
         const dim3 grid((unsigned)p.sblocks.size()), block(64 * kSumSplit);
         const float* corr = force ? (const float*)ws->corr.p : nullptr;
+        float4* const gpos = carry & kCarryOut ? ws->gpos.p : nullptr;
         if (pot)
-            hipLaunchKernelGGL(k_mutual_sum<true>, grid, block, 0, st, ws->sblocks.p, ws->sims.p, ws->rows.p,
+            hipLaunchKernelGGL(k_mutual_sum<true>, grid, block, 0, st, ws->sblocks.p, ws->sims.p,
                                64 * p.tiling.R, p.group_rows, ws->iside.p, ws->jside.p, ws->jintra.p, ws->gsum.p,
-                               corr, p.ntot, force, mpos, mvel, mv);
+                               corr, p.ntot, force, mpos, mvel, gpos, mv);
         else
-            hipLaunchKernelGGL(k_mutual_sum<false>, grid, block, 0, st, ws->sblocks.p, ws->sims.p, ws->rows.p,
+            hipLaunchKernelGGL(k_mutual_sum<false>, grid, block, 0, st, ws->sblocks.p, ws->sims.p,
                                64 * p.tiling.R, p.group_rows, ws->iside.p, ws->jside.p, ws->jintra.p, ws->gsum.p,
-                               corr, p.ntot, force, mpos, mvel, mv);
+                               corr, p.ntot, force, mpos, mvel, gpos, mv);
         GI_HIP(hipGetLastError());
     }
     if (timed) {
@@ -1154,11 +1199,11 @@ static void launch_contact(const Workspace* ws, float4* force, hipStream_t st) {
 // Full force evaluation for the current plan: grid, all pairs, finish (or
 // the direct pass alone).  With move_pos / move_vel (the arrays pos / vel
 // point to) and a plan with split_finish, the move is fused into the last
-// kernel and *moved is set; otherwise the caller moves.  The move takes each
-// simulation's own constants (the batched engine), or mv's when given.
+// kernel and *moved is set; otherwise the caller moves, and carry (of such a
+// fused move: PadCarry) has no effect.
 static int run_force(DevCtx* ctx, Workspace* ws, const float4* pos, const float4* vel, float4* force,
                      hipStream_t st, bool timed, float4* move_pos = nullptr, float4* move_vel = nullptr,
-                     bool* moved = nullptr, const SumMove* mv = nullptr) {
+                     bool* moved = nullptr, const SumMove& mv = SumMove{}, int carry = 0) {
     const Plan& p = ws->plan;
     if (p.ntot == 0) return 0;
     TimingPair whole;
@@ -1194,8 +1239,7 @@ static int run_force(DevCtx* ctx, Workspace* ws, const float4* pos, const float4
         if (p.split_finish) {
             const bool fuse = move_pos && move_vel && moved;
             if ((rc = launch_gravity(ctx, ws, pos, false, st, timed, force, ctx->ev_join, ctx->ev_fork, side_work,
-                                     fuse ? move_pos : nullptr, fuse ? move_vel : nullptr,
-                                     mv ? *mv : SumMove{0.0f, 0.0f, 0.0f, 1})))
+                                     fuse ? move_pos : nullptr, fuse ? move_vel : nullptr, mv, fuse ? carry : 0)))
                 return rc;
             if (fuse) *moved = true;
         } else {
@@ -2003,11 +2047,11 @@ static int impact_steps_impl(gi_float4* pos, gi_float4* vel, gi_float4* force, i
     key_append(key, m);
     // The move is fused into the force's last kernel when the plan allows
     // (k_move_collision's arithmetic, with these constants; nfe = NFe).
-    const SumMove smv{m.Dt, m.DtOverMassFe, m.DtOverMassSi, 0};
+    const SumMove smv{m.Dt, m.DtOverMassFe, m.DtOverMassSi, kMoveOne, 0, 0, 0, 0.0f, 0.0f};
     auto body = [&](hipStream_t cs, int steps) -> int {
         for (int k = 0; k < steps; ++k) {
             bool moved = false;
-            int r = run_force(ctx, &ctx->ws, P, V, F, cs, false, P, V, &moved, &smv);
+            int r = run_force(ctx, &ctx->ws, P, V, F, cs, false, P, V, &moved, smv, pad_carry(k, steps));
             if (r) return r;
             if (!moved)
                 hipLaunchKernelGGL(k_move_collision, dim3(nblk(n, 256)), dim3(256), 0, cs, P, V, (const float4*)F,
@@ -2167,13 +2211,19 @@ int gi_separate_steps(gi_float4* pos, gi_float4* vel, gi_float4* force, int n, c
     key_append(key, m);
     key_append(key, damp_rate_body1);
     key_append(key, damp_rate_body2);
+    // The damped move is fused into the force's last kernel when the plan
+    // allows (k_move_damped_separate's arithmetic).
+    const SumMove smv{m.Dt,       m.DtOverMassFe, m.DtOverMassSi,  kMoveDamped,    m.boarder1,
+                      m.boarder2, m.boarder3,     damp_rate_body1, damp_rate_body2};
     auto body = [&](hipStream_t cs, int steps) -> int {
         for (int k = 0; k < steps; ++k) {
-            int r = run_force(ctx, &ctx->ws, P, V, F, cs, false);
+            bool moved = false;
+            int r = run_force(ctx, &ctx->ws, P, V, F, cs, false, P, V, &moved, smv, pad_carry(k, steps));
             if (r) return r;
-            hipLaunchKernelGGL(k_move_damped_separate, dim3(nblk(n, 256)), dim3(256), 0, cs, P, V,
-                               (const float4*)F, n, m.Dt, m.DtOverMassFe, m.DtOverMassSi, m.boarder1, m.boarder2,
-                               m.boarder3, damp_rate_body1, damp_rate_body2);
+            if (!moved)
+                hipLaunchKernelGGL(k_move_damped_separate, dim3(nblk(n, 256)), dim3(256), 0, cs, P, V,
+                                   (const float4*)F, n, m.Dt, m.DtOverMassFe, m.DtOverMassSi, m.boarder1,
+                                   m.boarder2, m.boarder3, damp_rate_body1, damp_rate_body2);
             GI_HIP(hipGetLastError());
         }
         return 0;
@@ -2359,7 +2409,7 @@ int gi_ensemble_steps(gi_ensemble* e, int n_steps) {
                    [&](hipStream_t cs) -> int {
                        bool moved = false;
                        int r = run_force(ctx, &e->ws, e->pos, e->vel, e->force.p, cs, false, e->pos, e->vel,
-                                         &moved);
+                                         &moved, SumMove{0.0f, 0.0f, 0.0f, kMovePerSim, 0, 0, 0, 0.0f, 0.0f});
                        if (r) return r;
                        if (!moved)
                            hipLaunchKernelGGL(k_move, dim3(nblk(ntot, 256)), dim3(256), 0, cs, e->pos, e->vel,

@@ -70,9 +70,18 @@ struct RowDesc {
 };
 
 // One workgroup of k_mutual_sum: the 64 padded places [q0, q0 + 64) of
-// simulation sim (inside one row, as 64 divides the row length).
+// simulation sim (inside one row, as 64 divides the row length), the first
+// nreal of them particles i0 .. i0 + nreal - 1 of one material, with all that
+// their entries' addresses need, so that the workgroup's loads start after
+// one load instead of a chain of three: its row's slots, the groups before
+// its own and the rows before it in its group, the places of the block in
+// the first group's slab (jfirst) and in its group's first row (ifirst), and
+// the simulation's gn.
 struct SumBlock {
-    int sim, q0;
+    int sim, q0, i0, nreal;
+    int slot0, nslot, group, in_group;
+    long long jfirst, ifirst;
+    int gn, iron, pad0, pad1;
 };
 
 // Ghost position of the padded layout: every pair with a real particle has

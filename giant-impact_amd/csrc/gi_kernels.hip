@@ -195,6 +195,12 @@ __host__ __device__ __forceinline__ long long jside_row_offset(int row, int gn, 
     return (long long)row * gn - (long long)B * row * (row + 1) / 2;
 }
 
+// What group g of WB places adds to a place's entry offset over that of
+// group 0: SumBlock::jfirst + 3 times this is the place's record.
+__host__ __device__ __forceinline__ long long sum_group_offset(int g, int gn, long long WB) {
+    return (long long)g * gn - WB * g * (g + 1) / 2 - WB * g;
+}
+
 constexpr int kMutualWaves = 4;  // wavefronts per block of k_mutual
 
 // One wavefront's task t of simulation sd (P: its padded positions, q: the
@@ -585,65 +591,69 @@ __global__ void k_mutual_pad(const float4* __restrict__ pos, int gtot, const Sim
 // times the loads in flight of one thread per particle.
 // With corr (the contact corrections of k_contact_corr), the correction plus
 // the sum rounded to float goes to force.xyz -- k_finish's arithmetic --
-// and, with mpos / mvel, the particle then takes the move's step (k_move's
-// and k_move_collision's arithmetic) with the constants of mv, or with its
-// simulation's own when mv.per_sim; without corr, the sum goes to gsum for
-// k_finish / k_finish_potential.
+// and, with mpos / mvel, the particle then takes the move's step (k_move's,
+// k_move_collision's or k_move_damped_separate's arithmetic) with mv; with
+// gpos, the moved position also goes to its padded place, so that the next
+// step of the same run needs no k_mutual_pad (two separate bodies of 15,000
+// particles: 148.3 us a step with a move kernel and a padded copy of their
+// own, 142.6 fused; one simulation of 21,000, whose move was fused before,
+// 115 and 114).  Without corr, the sum goes to gsum for k_finish /
+// k_finish_potential.
+// Bound by the entries' bytes: 102 us at N = 262,144 (5.1 TB/s), 28 us at
+// 65,536.  Below, where a few loads in turn are all of it, one load of the
+// workgroup's descriptor instead of three in turn and the particle's state
+// asked for before the entries: 6.2 us -> 5.0 at N = 13,255.  Two or sixteen
+// entries in flight, or eight or sixteen wavefronts per block: the same
+// within 5% at every size.
 constexpr int kSumSplit = 4;
 
-// Move constants of a move fused into k_mutual_sum.
+// Move constants of a move fused into k_mutual_sum: one set for the call, or
+// each SimDesc's own (the batched engine), or the damped move's with its
+// borders (k_move_damped_separate).
+enum SumMoveKind { kMoveOne = 0, kMovePerSim = 1, kMoveDamped = 2 };
 struct SumMove {
     float dt, dt_over_mass_fe, dt_over_mass_si;
-    int per_sim;  // 1: take them from each SimDesc (the batched engine)
+    int kind;
+    int b1, b2, b3;
+    float damp1, damp2;
 };
 
-// Entries k0 .. k1 - 1 of one list (slots, or slab entries) added to
-// (sx, sy, sz) in order.  at(k) gives the wavefront-uniform address of entry
-// k's record for lane 0: lane l reads the (x, y, z) record at p + 3 l, so a
-// wavefront reads 768 contiguous bytes per entry.  The loads of kSumBatch
-// entries are issued before their additions, so a wavefront has that many
-// round trips to memory in flight instead of one; the additions keep their
-// order, so the sums are those of the one-at-a-time loop.  POT: x only.
-constexpr int kSumBatch = 4;
+// A wavefront's part of a particle's entries (its quarters of the slots, of
+// the earlier groups' slab entries and of the earlier rows of its group, one
+// after the other) are one list: the loads of kSumBatch entries are issued
+// before their additions, whatever list they are of, and so are those of the
+// entries left over, so a list costs one round trip to memory per kSumBatch
+// entries.  The additions keep their order.
+constexpr int kSumBatch = 8;
 
-template <bool POT, typename At>
-__device__ __forceinline__ void add_entries(int k0, int k1, int lane, At at, CompSum& sx, CompSum& sy,
-                                            CompSum& sz) {
-    int k = k0;
-    for (; k + kSumBatch <= k1; k += kSumBatch) {
-        float vx[kSumBatch], vy[kSumBatch], vz[kSumBatch];
+// Entries k .. k + M - 1: at(k)'s record holds lane 0's (x, y, z), lane l's
+// is 3 l further, so a wavefront reads 768 contiguous bytes per entry.  POT:
+// x only.
+template <int M, bool POT, typename At>
+__device__ __forceinline__ void add_entries(int k, int lane, At at, CompSum& sx, CompSum& sy, CompSum& sz) {
+    float vx[M], vy[M], vz[M];
 #pragma unroll
-        for (int u = 0; u < kSumBatch; ++u) {
-            const float* p = at(k + u) + 3 * lane;
-            vx[u] = p[0];
-            if constexpr (!POT) {
-                vy[u] = p[1];
-                vz[u] = p[2];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kSumBatch; ++u) {
-            sx.add(vx[u]);
-            if constexpr (!POT) {
-                sy.add(vy[u]);
-                sz.add(vz[u]);
-            }
+    for (int u = 0; u < M; ++u) {
+        const float* e = at(k + u) + 3 * lane;
+        vx[u] = e[0];
+        if constexpr (!POT) {
+            vy[u] = e[1];
+            vz[u] = e[2];
         }
     }
-    for (; k < k1; ++k) {
-        const float* p = at(k) + 3 * lane;
-        sx.add(p[0]);
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+        sx.add(vx[u]);
         if constexpr (!POT) {
-            sy.add(p[1]);
-            sz.add(p[2]);
+            sy.add(vy[u]);
+            sz.add(vz[u]);
         }
     }
 }
 
 template <bool POT>
 __global__ __launch_bounds__(64 * kSumSplit) void k_mutual_sum(const SumBlock* __restrict__ blocks,
-                                                              const SimDesc* __restrict__ sims,
-                                                              const RowDesc* __restrict__ rows, int B, int W,
+                                                              const SimDesc* __restrict__ sims, int B, int W,
                                                               const float* __restrict__ iside,
                                                               const float* __restrict__ jside,
                                                               const float* __restrict__ jintra,
@@ -651,47 +661,60 @@ __global__ __launch_bounds__(64 * kSumSplit) void k_mutual_sum(const SumBlock* _
                                                               const float* __restrict__ corr, int ntot,
                                                               float4* __restrict__ force,
                                                               float4* __restrict__ mpos,
-                                                              float4* __restrict__ mvel, SumMove mv) {
+                                                              float4* __restrict__ mvel,
+                                                              float4* __restrict__ gpos, SumMove mv) {
     __shared__ float red[3][2][kSumSplit][64];  // per component: sum and compensation of each quarter
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: the addresses below stay scalar
     const SumBlock blk = blocks[blockIdx.x];
-    const SimDesc& sd = sims[blk.sim];
-    const int q = blk.q0 + lane;
-    const int row = blk.q0 / B;
-    const int o0 = blk.q0 - row * B;  // lane 0's place in its row
-    // the particle at padded place q, or -1 for a ghost
-    int i = -1;
-    if (q < sd.gfe) {
-        if (q < sd.fe_end - sd.start) i = sd.start + q;
-    } else if (q - sd.gfe < sd.end - sd.fe_end) {
-        i = sd.fe_end + (q - sd.gfe);
+    const bool real = lane < blk.nreal;
+    const int i = blk.i0 + lane;
+    // what the last step needs, on its way beside the entries
+    float2 rx = {}, ry = {}, rz = {};
+    float4 v = {}, p = {};
+    if (w == 0 && real && corr) {
+        const float2* rec = reinterpret_cast<const float2*>(corr + 6 * (size_t)i);
+        rx = rec[0];
+        ry = rec[1];
+        rz = rec[2];
+        if (mpos) {
+            v = mvel[i];
+            p = mpos[i];
+        }
     }
     CompSum sx, sy, sz;
     sx.zero();
     sy.zero();
     sz.zero();
-    if (i >= 0) {
-        const RowDesc rd = rows[sd.row0 + row];
-        add_entries<POT>(
-            rd.nslot * w / kSumSplit, rd.nslot * (w + 1) / kSumSplit, lane,
-            [&](int k) { return iside + (size_t)(rd.slot0 + k) * (3 * B) + 3 * o0; },
-            sx, sy, sz);
-        // the j-side entries of the earlier groups of W rows (W = 1: rows) ...
-        const int group = row / W, WB = W * B;
-        add_entries<POT>(
-            group * w / kSumSplit, group * (w + 1) / kSumSplit, lane,
-            [&](int r) {
-                return jside + sd.jbase + 3 * (jside_row_offset(r, sd.gn, WB) + (blk.q0 - (long long)(r + 1) * WB));
-            },
-            sx, sy, sz);
-        // ... and of the earlier rows of its own group
-        const int in_group = row - group * W;
-        const long long ilen = (long long)(W - 1) * B;
-        add_entries<POT>(
-            group * W + in_group * w / kSumSplit, group * W + in_group * (w + 1) / kSumSplit, lane,
-            [&](int r) { return jintra + sd.jibase + 3 * (ilen * r + (blk.q0 - (long long)(r + 1) * B)); },
-            sx, sy, sz);
+    const int sl0 = blk.nslot * w / kSumSplit, gr0 = blk.group * w / kSumSplit, in0 = blk.in_group * w / kSumSplit;
+    const int nsl = blk.nslot * (w + 1) / kSumSplit - sl0;
+    const int nsg = nsl + blk.group * (w + 1) / kSumSplit - gr0;
+    const int n = nsg + blk.in_group * (w + 1) / kSumSplit - in0;
+    const float* const slots = iside + (size_t)(blk.slot0 + sl0) * (3 * B) + 3 * (blk.q0 % B);
+    const float* const groups = jside + blk.jfirst;
+    const long long istep = 3 * ((long long)(W - 1) * B - B);
+    const float* const inner = jintra + blk.ifirst + istep * in0;
+    // the record of entry k for lane 0 (wavefront-uniform); lane l's is 3 l further
+    auto at = [&](int k) {
+        const float* const a0 = slots + (size_t)k * (3 * B);
+        const float* const a1 = groups + 3 * sum_group_offset(gr0 + k - nsl, blk.gn, (long long)W * B);
+        const float* const a2 = inner + istep * (k - nsg);
+        const float* const a12 = k < nsg ? a1 : a2;
+        return k < nsl ? a0 : a12;
+    };
+    if (real) {
+        int k = 0;
+        for (; k + kSumBatch <= n; k += kSumBatch) add_entries<kSumBatch, POT>(k, lane, at, sx, sy, sz);
+        switch (n - k) {
+            case 7: add_entries<7, POT>(k, lane, at, sx, sy, sz); break;
+            case 6: add_entries<6, POT>(k, lane, at, sx, sy, sz); break;
+            case 5: add_entries<5, POT>(k, lane, at, sx, sy, sz); break;
+            case 4: add_entries<4, POT>(k, lane, at, sx, sy, sz); break;
+            case 3: add_entries<3, POT>(k, lane, at, sx, sy, sz); break;
+            case 2: add_entries<2, POT>(k, lane, at, sx, sy, sz); break;
+            case 1: add_entries<1, POT>(k, lane, at, sx, sy, sz); break;
+            default: break;
+        }
     }
     red[0][0][w][lane] = sx.s;
     red[0][1][w][lane] = sx.c;
@@ -700,7 +723,7 @@ __global__ __launch_bounds__(64 * kSumSplit) void k_mutual_sum(const SumBlock* _
     red[2][0][w][lane] = sz.s;
     red[2][1][w][lane] = sz.c;
     __syncthreads();
-    if (w == 0 && i >= 0) {
+    if (w == 0 && real) {
         // the quarters in order; their compensations join the total's
         CompSum ax, ay, az;
         ax.zero();
@@ -718,8 +741,6 @@ __global__ __launch_bounds__(64 * kSumSplit) void k_mutual_sum(const SumBlock* _
         if (corr) {
             // k_finish's arithmetic: the correction's (sum, compensation)
             // pair plus the all-pairs sum rounded to float, rounded once
-            const float2* rec = reinterpret_cast<const float2*>(corr + 6 * (size_t)i);
-            const float2 rx = rec[0], ry = rec[1], rz = rec[2];
             CompSum cx{rx.x, rx.y}, cy{ry.x, ry.y}, cz{rz.x, rz.y};
             cx.add(ax.value());
             cy.add(ay.value());
@@ -729,20 +750,30 @@ __global__ __launch_bounds__(64 * kSumSplit) void k_mutual_sum(const SumBlock* _
             force[i].y = fy;
             force[i].z = fz;
             if (mpos) {
-                const float dt = mv.per_sim ? sd.dt : mv.dt;
-                const float dtm_fe = mv.per_sim ? sd.dt_over_mass_fe : mv.dt_over_mass_fe;
-                const float dtm_si = mv.per_sim ? sd.dt_over_mass_si : mv.dt_over_mass_si;
-                const float temp = i < sd.fe_end ? dtm_fe : dtm_si;
-                float4 v = mvel[i];
-                float4 p = mpos[i];
-                v.x += fx * temp;
-                v.y += fy * temp;
-                v.z += fz * temp;
+                const SimDesc& sd = sims[blk.sim];
+                const bool own = mv.kind == kMovePerSim;
+                const float dt = own ? sd.dt : mv.dt;
+                const float dtm_fe = own ? sd.dt_over_mass_fe : mv.dt_over_mass_fe;
+                const float dtm_si = own ? sd.dt_over_mass_si : mv.dt_over_mass_si;
+                if (mv.kind == kMoveDamped) {
+                    const bool second = mv.b3 <= i || mv.b2 <= i;
+                    const bool si = mv.b3 <= i || (mv.b2 > i && mv.b1 <= i);
+                    const float temp = si ? dtm_si : dtm_fe, damp = second ? mv.damp2 : mv.damp1;
+                    v.x += (fx - damp * v.x) * temp;
+                    v.y += (fy - damp * v.y) * temp;
+                    v.z += (fz - damp * v.z) * temp;
+                } else {
+                    const float temp = blk.iron ? dtm_fe : dtm_si;
+                    v.x += fx * temp;
+                    v.y += fy * temp;
+                    v.z += fz * temp;
+                }
                 p.x += v.x * dt;
                 p.y += v.y * dt;
                 p.z += v.z * dt;
                 mvel[i] = v;
                 mpos[i] = p;
+                if (gpos) gpos[sd.gbase + blk.q0 + lane] = p;
             }
         } else {
             gsum[i] = make_float4(ax.value(), ay.value(), az.value(), 0.0f);
