@@ -5,8 +5,8 @@
 //              rcp (1 multiply, 2 transcendental ops); 2 = mutual pass (each
 //              pair once for both particles, rows of 64*R, rsq cubed);
 //              3 = direct pass (small simulations: the whole force in one
-//              launch; R = lanes per i-particle, 1, 2 or 4 (8 acts as 4),
-//              64 / R i-particles per workgroup; the sizes unused);
+//              launch; 64 / R i-particles per workgroup, R = 1, 2, 4 or 8;
+//              the sizes unused);
 //              4 = mutual pass with row groups (a workgroup's four
 //              wavefronts hold four rows and add their j-side sums in LDS
 //              before writing them: a quarter of the j-side slab; R = 4 or 8)
@@ -25,6 +25,7 @@
 
 #include <dlfcn.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -135,10 +136,14 @@ inline BatchedTiling batched_tiling() {
     return BatchedTiling{4096, 1, 0};
 }
 
+// The row for a launch of ntot particles.  Several simulations in one launch
+// (the separate bodies) have the work of one with as many pairs, sum n^2,
+// and are placed by that size: two of 8,000 (11,314) step in 59 us by the
+// direct pass's row and in 66 by the row of 16,000; two of 18,000 (25,456)
+// in 140 and, by the row of 36,000, 159.
 inline Tiling choose_tiling(long long ntot, long long pairs, int nsims) {
-    (void)pairs;
-    (void)nsims;
     if (tiling_override().active) return tiling_override().t;
+    if (nsims > 1) ntot = (long long)std::ceil(std::sqrt((double)pairs));
     for (const TuningRow& r : tuning_table())
         if (ntot <= r.n_max) return r.t;
     Tiling t{4, 0, 0, 8192, 512};

@@ -34,9 +34,9 @@ CLASSES = [
     (3072, 1536, 512),
     (6144, 3072, 1024),
     (12288, 6144, 2048),
-    (16384, 10752, 3584),
-    (24576, 15360, 5120),
-    (49152, 24576, 8192),
+    (27648, 13312, 4435),
+    (33792, 24576, 6144),
+    (49152, 31488, 10496),
     (98304, 49152, 16384),
     (196608, 98304, 32768),
     (393216, 196608, 65536),
@@ -126,7 +126,7 @@ def main(argv=None) -> int:
     # at N = 262,144); --variants sweeps it again
     variants = [0, 1] if args.variants else [0]
     targets = [4096, 8192, 16384, 32768, 65536, 131072] if not args.quick else [32768]
-    mutual_Ls = [192, 256, 384, 512, 768, 1024, 1536, 2048] if not args.quick else [512]
+    mutual_Ls = [128, 192, 256, 384, 512, 768, 1024, 1536, 2048] if not args.quick else [512]
     rows = []
     only = {int(x) for x in args.classes.split(",") if x.strip()}
     kept = {}
