@@ -1341,20 +1341,22 @@ static int launch_recenter(DevCtx* ctx, float4* pos, float4* vel, int n, int nfe
 static int recenter_ref_scratch(DevCtx* ctx, int n, RcWork* wk) {
     wk->window = 64;
     while (nblk(n, wk->window) > kRcMaxRuns) wk->window *= 2;
-    const size_t w = wk->nwin = nblk(n, wk->window);
+    const size_t w = wk->nwin = nblk(n, wk->window), groups = wk->ngroups = nblk(wk->nwin, kRcGroup);
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t o = at;
         at = (at + bytes + 255) / 256 * 256;
         return o;
     };
-    const size_t runs = take(kRcChains * w * kRcStarts * sizeof(RcRun)), sums = take(kRcChains * w * sizeof(double)),
+    const size_t runs = take(kRcChains * w * kRcStarts * sizeof(RcRun)),
+                 joined = take(kRcChains * groups * kRcStarts * sizeof(RcRun)), sums = take(kRcChains * w * sizeof(double)),
                  bound = take(kRcChains * (w + 1) * sizeof(int)), guess = take(kRcChains * w * sizeof(float)),
                  total = take(kRcChains * sizeof(float));
     int rc = ctx->rc_ref.ensure(at);
     if (rc) return rc;
     unsigned char* p = ctx->rc_ref.p;
     wk->runs = (RcRun*)(p + runs);
+    wk->groups = (RcRun*)(p + joined);
     wk->sums = (double*)(p + sums);
     wk->bound = (int*)(p + bound);
     wk->guess = (float*)(p + guess);
@@ -1373,9 +1375,8 @@ static int launch_recenter_ref(DevCtx* ctx, float4* pos, float4* vel, int n, int
     const dim3 wgrid(nblk(wk.nwin, kRcWindowWaves)), wblock(64 * kRcWindowWaves);
     hipLaunchKernelGGL(k_rc_window_sums, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
     hipLaunchKernelGGL(k_rc_bounds, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
-    hipLaunchKernelGGL(k_rc_runs, dim3(nblk((long long)kRcChains * wk.nwin * kRcStarts, 256)), dim3(256), 0, st, P, V,
-                       nfe, mfe, msi, wk);
-    hipLaunchKernelGGL(k_rc_join, dim3(kRcChains), dim3(kRcJoinThreads), 0, st, P, V, nfe, mfe, msi, wk);
+    hipLaunchKernelGGL(k_rc_runs, dim3(kRcChains * wk.ngroups), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
+    hipLaunchKernelGGL(k_rc_join, dim3(kRcChains), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
     hipLaunchKernelGGL(k_recenter_ref_apply, dim3(nblk(n, 256)), dim3(256), 0, st, pos, vel, n,
                        (const float*)wk.total, tc[0], tc[1], tc[2], tv[0], tv[1], tv[2]);
     GI_HIP(hipGetLastError());

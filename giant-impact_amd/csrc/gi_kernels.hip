@@ -1837,25 +1837,30 @@ __global__ void k_recenter_apply(float4* __restrict__ pos, float4* __restrict__ 
 //                      the start matter) and guesses the start from it;
 //   k_rc_runs          every run from 16 starts, one float ulp apart (they
 //                      cover every residue up to 8 ulps), with its largest
-//                      binade and least distance;
-//   k_rc_join          one workgroup per chain: runs joined in groups of 16
-//                      from the group's 16 starts side by side, then the
-//                      groups in order from the true start; where the
-//                      conditions do not hold, run by run, and a run that
-//                      does not hold is taken step by step.  No result
-//                      depends on a guess: a guess only decides which way it
-//                      is reached.
+//                      binade and least distance; then a workgroup's 16 runs
+//                      joined from its first run's 16 starts;
+//   k_rc_join          one wavefront per chain: the joined groups in order
+//                      from the true start; where the conditions do not
+//                      hold, run by run, and a run that does not hold is
+//                      taken step by step.  No result depends on a guess: a
+//                      guess only decides which way it is reached.
+// Joining looks at all 16 starts at once, one per lane of a row, and takes the
+// first that holds: a third fewer groups go run by run than with the one
+// start picked by the difference, and nothing is looked up by it (0.24 us a
+// group or run instead of 0.28, and the groups' own joins, 11 us in the
+// chains' seven workgroups, run beside the others).
 // Bound by the join's chain of dependent FP64 operations.  The impact states
-// need 0 to 9 of 1,024 runs step by step.  N = 65,536: 122 us a call (sums
-// 5 us, bounds 18, runs 23, join 50 to 110, apply 5) against 3,404 step by
-// step; windows of 128 took 135.
+// need 0 to 14 of 1,024 runs step by step.  N = 65,536: 105 us a call (sums
+// 5 us, bounds 17, runs 28, join 45 to 77, apply 5; 122 us with the groups
+// joined in the chains' own workgroups and one start tried) against 3,404
+// step by step; windows of 128 took 135.
 constexpr int kRcChains = 7;
 constexpr int kRcStarts = 16;
 constexpr int kRcGroup = 16;     // runs per group
 constexpr int kRcMaxRuns = 1024;
 constexpr float kRcRoom = 1.0e30f;  // no step yet
-constexpr int kRcJoinThreads = kRcMaxRuns / kRcGroup * kRcStarts;
-static_assert(kRcJoinThreads <= 1024, "one workgroup joins a chain");
+constexpr int kRcMaxGroups = kRcMaxRuns / kRcGroup;
+static_assert(kRcStarts == 16 && kRcGroup == 16, "a workgroup of 256 holds a group's runs; a row of lanes a run's starts");
 
 // A run from one start: its end, the least distance of a sum from its
 // binade's ends (negative: never shift this run) and the largest binade.
@@ -1872,8 +1877,9 @@ struct RcWork {
     int* bound;     // [kRcChains][nwin + 1]
     float* guess;   // [kRcChains][nwin]
     RcRun* runs;    // [kRcChains][nwin][kRcStarts]
+    RcRun* groups;  // [kRcChains][ngroups][kRcStarts]: kRcGroup runs joined; binade -1: they do not hold
     float* total;   // [kRcChains]
-    int window, nwin;
+    int window, nwin, ngroups;
 };
 
 // Term k of chain c: x, y, z, vx, vy, vz, 1 times the element's mass.
@@ -2034,112 +2040,116 @@ __device__ __forceinline__ void rc_step(float& a, float x, double t, int& binade
     a = (float)s;
 }
 
+// Whether run (or group) r, taken from `start`, holds for the true start a,
+// and the difference d of the two.
+__device__ __forceinline__ bool rc_holds(float a, float start, const RcRun& r, double& d) {
+    d = (double)a - (double)start;
+    const double k = __builtin_amdgcn_ldexp(d, 1023 + 22 - r.binade);  // in pairs of ulps of the run's largest binade
+    const bool exact = (double)a - d == (double)start;
+    const bool shift = fabs(d) < (double)r.room && k == rint(k);
+    // binade 0: every term is zero
+    return exact && (d == 0.0 || r.binade == 0 || shift) && r.binade >= 0;
+}
+
+// Lane j of a row of 16 holds a run's (or group's) start j and what it led
+// to: the lowest lane of the row it holds for, or -1.  All rows of the
+// wavefront take part.
+__device__ __forceinline__ int rc_pick(bool holds, int lane) {
+    const unsigned m = (unsigned)(__ballot(holds) >> (lane & 48)) & 0xffffu;
+    return m ? (lane & 48) + __builtin_ctz(m) : -1;
+}
+
+// One workgroup per group of a chain: the group's runs from their starts, a
+// run and start per lane, then the runs joined from each of the group's
+// starts, a row of lanes per start.
 __global__ __launch_bounds__(256) void k_rc_runs(const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                  int nfe, double mass_fe, double mass_si, RcWork wk) {
-    const int id = blockIdx.x * 256 + threadIdx.x;
-    const int j = id % kRcStarts, s = id / kRcStarts % wk.nwin, c = id / kRcStarts / wk.nwin;
-    if (c >= kRcChains) return;
-    const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
-    const int b = bound[s], e = bound[s + 1];
-    RcRun r{rc_start(wk.guess[c * wk.nwin + s], j), 0, kRcRoom, 0};
-    float x[8], nx[8];
+    __shared__ RcRun run[kRcGroup][kRcStarts];
+    __shared__ float guess[kRcGroup];
+    const int c = blockIdx.x / wk.ngroups, g = blockIdx.x % wk.ngroups;
+    const int row = threadIdx.x / kRcStarts, j = threadIdx.x % kRcStarts, lane = threadIdx.x & 63;
+    const int s0 = g * kRcGroup, ns = min(kRcGroup, wk.nwin - s0);
+    if (row < ns) {
+        const int s = s0 + row;
+        const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
+        const int b = bound[s], e = bound[s + 1];
+        const float gs = wk.guess[c * wk.nwin + s];
+        if (j == 0) guess[row] = gs;
+        RcRun r{rc_start(gs, j), 0, kRcRoom, 0};
+        float x[8], nx[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = rc_value(pos, vel, c, min(b + u, e - 1));
-    for (int k = b; k < e; k += 8) {
+        for (int u = 0; u < 8; ++u) x[u] = rc_value(pos, vel, c, min(b + u, e - 1));
+        for (int k = b; k < e; k += 8) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) nx[u] = rc_value(pos, vel, c, min(k + 8 + u, e - 1));
+            for (int u = 0; u < 8; ++u) nx[u] = rc_value(pos, vel, c, min(k + 8 + u, e - 1));
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (k + u < e) rc_step(r.end, x[u], (double)x[u] * (k + u < nfe ? mass_fe : mass_si), r.binade, r.room);
+            for (int u = 0; u < 8; ++u)
+                if (k + u < e) rc_step(r.end, x[u], (double)x[u] * (k + u < nfe ? mass_fe : mass_si), r.binade, r.room);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = nx[u];
+            for (int u = 0; u < 8; ++u) x[u] = nx[u];
+        }
+        wk.runs[((size_t)c * wk.nwin + s) * kRcStarts + j] = r;
+        run[row][j] = r;
     }
-    wk.runs[((size_t)c * wk.nwin + s) * kRcStarts + j] = r;
+    __syncthreads();
+    RcRun x{rc_start(guess[0], row), 0, kRcRoom, 0};
+    for (int s = 0; s < ns; ++s) {
+        const RcRun r = run[s][j];
+        double d;
+        const int at = rc_pick(rc_holds(x.end, rc_start(guess[s], j), r, d), lane);
+        const int from = max(at, 0);
+        // rounded down: the least factor below 1 takes more than the
+        // subtraction's and the conversion's rounding
+        const float room = (float)(((double)r.room - fabs(d)) * (1.0 - 0x1p-20));
+        x.end = __shfl((float)((double)r.end + d), from);
+        x.room = fminf(x.room, __shfl(room, from));
+        const int binade = __shfl(r.binade, from);
+        x.binade = x.binade < 0 || at < 0 ? -1 : max(x.binade, binade);
+    }
+    if (j == 0) wk.groups[((size_t)c * wk.ngroups + g) * kRcStarts + row] = x;
 }
 
-// The start of a run or group guessed at g that the true start `a` differs
-// from by a multiple of kRcStarts ulps, and that difference.
-struct RcShift {
-    int j;
-    double d;
-    bool exact;
-};
-__device__ __forceinline__ RcShift rc_shift(float a, float g) {
-    const int e = (int)((__float_as_uint(g) >> 23) & 0xff);
-    RcShift x{0, 0.0, false};
-    const double k = __builtin_amdgcn_ldexp((double)a - (double)g, 127 + 23 - e);  // in ulps of g
-    if (e != 0 && e != 255 && fabs(k) < 1.0e9) x.j = (int)rint(k) & (kRcStarts - 1);
-    const float s = rc_start(g, x.j);
-    x.d = (double)a - (double)s;
-    x.exact = (double)a - x.d == (double)s;
-    return x;
-}
-// Whether a run holds when its start is shifted by d.
-__device__ __forceinline__ bool rc_holds(const RcShift& x, int binade, float room) {
-    if (!x.exact) return false;
-    if (x.d == 0.0 || binade == 0) return true;  // binade 0: every term is zero
-    if (!(fabs(x.d) < (double)room)) return false;
-    const double k = __builtin_amdgcn_ldexp(x.d, 1023 + 22 - binade);  // in pairs of ulps
-    return k == rint(k);
-}
-__device__ __forceinline__ float rc_shifted(const RcRun& r, const RcShift& h) { return (float)((double)r.end + h.d); }
-
-__global__ __launch_bounds__(kRcJoinThreads) void k_rc_join(const float4* __restrict__ pos,
-                                                            const float4* __restrict__ vel, int nfe, double mass_fe,
-                                                            double mass_si, RcWork wk) {
-    __shared__ RcRun group[kRcJoinThreads];
-    __shared__ RcRun one[kRcGroup * kRcStarts];  // the runs of a group that does not hold
+__global__ __launch_bounds__(256) void k_rc_join(const float4* __restrict__ pos, const float4* __restrict__ vel,
+                                                 int nfe, double mass_fe, double mass_si, RcWork wk) {
+    __shared__ RcRun group[kRcMaxGroups][kRcStarts];
+    __shared__ RcRun one[kRcGroup][kRcStarts];  // the runs of a group that does not hold
     __shared__ float guess[kRcMaxRuns];
     __shared__ double terms[64];
     const int c = blockIdx.x;
     const RcRun* __restrict__ runs = wk.runs + (size_t)c * wk.nwin * kRcStarts;
-    const int ngroups = (wk.nwin + kRcGroup - 1) / kRcGroup;
-    const int g = threadIdx.x / kRcStarts, j = threadIdx.x % kRcStarts;
-    for (int s = threadIdx.x; s < wk.nwin; s += kRcJoinThreads) guess[s] = wk.guess[c * wk.nwin + s];
-    __syncthreads();
-    if (g < ngroups) {
-        RcRun x{rc_start(guess[g * kRcGroup], j), 0, kRcRoom, 0};
-        for (int s = g * kRcGroup; s < min((g + 1) * kRcGroup, wk.nwin); ++s) {
-            const RcShift h = rc_shift(x.end, guess[s]);
-            const RcRun r = runs[s * kRcStarts + h.j];
-            if (!rc_holds(h, r.binade, r.room)) {
-                x.binade = -1;
-                break;
-            }
-            x.end = rc_shifted(r, h);
-            x.binade = max(x.binade, r.binade);
-            // rounded down: the least factor below 1 takes more than the
-            // subtraction's and the conversion's rounding
-            x.room = fminf(x.room, (float)(((double)r.room - fabs(h.d)) * (1.0 - 0x1p-20)));
-        }
-        group[threadIdx.x] = x;
-    }
+    const int ngroups = wk.ngroups;
+    for (int s = threadIdx.x; s < wk.nwin; s += 256) guess[s] = wk.guess[c * wk.nwin + s];
+    for (int k = threadIdx.x; k < ngroups * kRcStarts; k += 256)
+        group[0][k] = wk.groups[(size_t)c * ngroups * kRcStarts + k];
     __syncthreads();
     if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x, j = lane % kRcStarts;
     const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
     float a = 0.0f;
+    // a joined with run (or group) r from start guess gs: whether it holds
+    auto take = [&](const RcRun& r, float gs) {
+        double d;
+        const unsigned m = (unsigned)__ballot(rc_holds(a, rc_start(gs, j), r, d)) & 0xffffu;  // the rows agree
+        if (!m) return false;
+        a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int((float)((double)r.end + d)), __builtin_ctz(m)));
+        return true;
+    };
+    RcRun r = group[0][j];
+    float gs = guess[0];
     for (int q = 0; q < ngroups; ++q) {
-        {
-            const RcShift h = rc_shift(a, guess[q * kRcGroup]);
-            const RcRun r = group[q * kRcStarts + h.j];
-            if (r.binade >= 0 && rc_holds(h, r.binade, r.room)) {
-                a = rc_shifted(r, h);
-                continue;
-            }
-        }
+        const RcRun nr = group[min(q + 1, ngroups - 1)][j];  // the next group's, on its way
+        const float ngs = guess[min(q + 1, ngroups - 1) * kRcGroup];
+        const bool held = take(r, gs);
+        r = nr;
+        gs = ngs;
+        if (held) continue;
         const int s0 = q * kRcGroup, s1 = min(s0 + kRcGroup, wk.nwin);
         wave_lds_sync();
-        for (int k = lane; k < (s1 - s0) * kRcStarts; k += 64) one[k] = runs[s0 * kRcStarts + k];
+        for (int k = lane; k < (s1 - s0) * kRcStarts; k += 64) one[0][k] = runs[s0 * kRcStarts + k];
         const int edge = bound[min(s0 + lane, wk.nwin)];  // lanes 0..kRcGroup
         wave_lds_sync();
         for (int s = s0; s < s1; ++s) {
-            const RcShift h = rc_shift(a, guess[s]);
-            const RcRun r = one[(s - s0) * kRcStarts + h.j];
-            if (rc_holds(h, r.binade, r.room)) {
-                a = rc_shifted(r, h);
-                continue;
-            }
+            if (take(one[s - s0][j], guess[s])) continue;
             const int e = __shfl(edge, s + 1 - s0);
             for (int k0 = __shfl(edge, s - s0); k0 < e; k0 += 64) {
                 wave_lds_sync();
