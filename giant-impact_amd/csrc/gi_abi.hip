@@ -302,12 +302,13 @@ constexpr long long kMutualMaxChunk = 4096;
 // sixteenth gained less).
 //
 // The divisor: a small company's step lasts as long as its longest tasks, a
-// large one's is the longer the more slots there are.  At 32 throughout,
-// eight simulations of 4,000 to 18,600 particles step in 0.279 ms, four of
-// 12,300 to 18,000 in 0.312; as below 0.238 and 0.258, and the 64-simulation
-// ensemble the same (4.64 ms; 1.1% slower at 64 throughout).  One of 30,000
-// is 2% faster at 32 than at 48.
-static long long batched_piece_div(long long n) { return n <= 12288 ? 64 : n <= 24576 ? 48 : 32; }
+// large one's is the longer the more slots there are.  At 32 throughout (and
+// the lists dealt out as below), eight simulations of 4,000 to 18,600
+// particles step in 256 us, two of up to 16,000 in 172, two of 9,500 in 114,
+// four of 12,300 to 18,000 in 260; as below 220, 100, 88 and 231, and the
+// 64-simulation ensemble the same (4.60 ms; 0.5% slower at 64 throughout).
+// One of 30,000 is 2% faster at 32 than at 48.
+static long long batched_piece_div(long long n) { return n <= 16384 ? 80 : n <= 24576 ? 48 : 32; }
 constexpr long long kTailPieces = 1536;
 constexpr long long kBatchedTailDiv = 8;
 

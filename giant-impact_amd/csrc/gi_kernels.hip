@@ -1845,10 +1845,10 @@ __global__ void k_recenter_apply(float4* __restrict__ pos, float4* __restrict__ 
 //                      taken step by step.  No result depends on a guess: a
 //                      guess only decides which way it is reached.
 // Joining looks at all 16 starts at once, one per lane of a row, and takes the
-// first that holds: a third fewer groups go run by run than with the one
-// start picked by the difference, and nothing is looked up by it (0.24 us a
-// group or run instead of 0.28, and the groups' own joins, 11 us in the
-// chains' seven workgroups, run beside the others).
+// first that holds: 24 groups of an impact state's 448 go run by run instead
+// of the 27 where only the start picked by the difference was tried, nothing
+// is looked up by it (0.24 us a group or run instead of 0.28), and the
+// groups' own joins, 11 us in the chains' seven workgroups, run side by side.
 // Bound by the join's chain of dependent FP64 operations.  The impact states
 // need 0 to 14 of 1,024 runs step by step.  N = 65,536: 105 us a call (sums
 // 5 us, bounds 17, runs 28, join 45 to 77, apply 5; 122 us with the groups
