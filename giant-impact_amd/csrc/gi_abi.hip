@@ -589,6 +589,15 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
     return 0;
 }
 
+// Wavefronts per workgroup of k_direct for n particles (of all simulations):
+// up to 2,048 particles there is a workgroup per CU at most, and 16
+// wavefronts shorten its chain (a step of N = 2,048 takes 9.8 us against 10.2
+// with 8); above, 8 leave room for the next workgroup beside the running ones
+// (N = 3,000 13.1 against 15.4 us, 4,096 15.2 against 17.9, 11,000 53 against
+// 69; four wavefronts were slower up to 8,192 and even above).
+constexpr long long kDirectWideMaxN = 2048;
+static int direct_waves(long long n) { return n <= kDirectWideMaxN ? 16 : 8; }
+
 // The plan of one force evaluation over `sims`: the mutual pass's tasks and
 // rows for the simulations that take it, then the one-sided pass's chunks
 // and tasks for the rest, the contact-grid bucket ranges and the moment
@@ -633,7 +642,10 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
         for (size_t si = 0; si < sims.size(); ++si)
             if (sims[si].active)
                 for (int i0 = sims[si].start; i0 < sims[si].end; i0 += ib)
-                    p.dblocks.push_back(DirectBlock{(int)si, i0, sims[si].start, sims[si].fe_end, sims[si].end, 0, 0, 0});
+                    p.dblocks.push_back(DirectBlock{(int)si, i0, sims[si].start, sims[si].fe_end, sims[si].end,
+                                                    direct_iron_waves(sims[si].start, sims[si].fe_end, sims[si].end,
+                                                                      direct_waves(ntot)),
+                                                    0, 0});
         p.direct = true;
     }
     long long pbase = 0;
@@ -1132,15 +1144,6 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
     return 0;
 }
 
-// Wavefronts per workgroup of k_direct for n particles (of all simulations):
-// up to 2,048 particles there is a workgroup per CU at most, and 16
-// wavefronts shorten its chain (a step of N = 2,048 takes 9.8 us against 10.2
-// with 8); above, 8 leave room for the next workgroup beside the running ones
-// (N = 3,000 13.1 against 15.4 us, 4,096 15.2 against 17.9, 11,000 53 against
-// 69; four wavefronts were slower up to 8,192 and even above).
-constexpr long long kDirectWideMaxN = 2048;
-static int direct_waves(long long n) { return n <= kDirectWideMaxN ? 16 : 8; }
-
 // k_direct over a block table of 64 / lanes i-particles per entry.
 template <int MOVE>
 static void direct_kernel(int lanes, int waves, int nblocks, hipStream_t st, const float4* pos, const float4* vel,
@@ -1574,10 +1577,10 @@ static NoAllocScratch* g_noalloc_ptr[64];  // per device, set once
 
 // Writes the descriptor and the block table of one simulation of n
 // particles, ib i-particles per workgroup.
-__global__ void k_noalloc_plan(NoAllocScratch* __restrict__ s, SimDesc sd, int nb, int ib) {
+__global__ void k_noalloc_plan(NoAllocScratch* __restrict__ s, SimDesc sd, int nb, int ib, int iron_waves) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) s->sim = sd;
-    if (b < nb) s->blocks[b] = DirectBlock{0, b * ib, sd.start, sd.fe_end, sd.end, 0, 0, 0};
+    if (b < nb) s->blocks[b] = DirectBlock{0, b * ib, sd.start, sd.fe_end, sd.end, iron_waves, 0, 0};
 }
 
 }  // namespace gi
@@ -1853,7 +1856,7 @@ int gi_force_collision_noalloc(const gi_float4* pos, const gi_float4* vel, gi_fl
                          kNoAllocMaxBlocks);
     hipStream_t st = as_stream(stream);
     hipLaunchKernelGGL(k_noalloc_plan, dim3(nblk(nb, 256)), dim3(256), 0, st, sp, make_sim(0, c->NFe, n, law_of(c)),
-                       nb, ib);
+                       nb, ib, direct_iron_waves(0, c->NFe, n, direct_waves(n)));
     direct_kernel<0>(lanes, direct_waves(n), nb, st, (const float4*)pos, (const float4*)vel, sp->blocks, &sp->sim,
                      (float4*)force, FusedMove{});
     GI_HIP(hipGetLastError());

@@ -59,10 +59,20 @@ struct GroupTask {
 
 // 64 / R i-particles from i0 on of simulation sim in the direct pass (the
 // last block of a simulation may be ragged), with the simulation's ranges
-// beside them: a workgroup starts from one load, not two in turn.
+// beside them, and how many wavefronts of a workgroup take iron j: a
+// workgroup starts from one load, not two in turn, and divides nothing.
 struct DirectBlock {
-    int sim, i0, start, fe_end, end, pad0, pad1, pad2;
+    int sim, i0, start, fe_end, end, iron_waves, pad0, pad1;
 };
+// The share of W wavefronts that takes a simulation's iron 64-blocks of j; at
+// least one for each material there is.
+__host__ __device__ __forceinline__ int direct_iron_waves(int start, int fe_end, int end, int W) {
+    const int bf = (fe_end - start + 63) >> 6, bs = (end - fe_end + 63) >> 6;
+    if (bf == 0) return 0;
+    if (bs == 0) return W;
+    const int w = (2 * W * bf + bf + bs) / (2 * (bf + bs));
+    return w < 1 ? 1 : w > W - 1 ? W - 1 : w;
+}
 
 // The i-side slots of one row: slot0 .. slot0 + nslot - 1, in task order.
 struct RowDesc {

@@ -1146,8 +1146,8 @@ __global__ __launch_bounds__(64 * kContactWaves) void k_contact_corr(int ntot, c
 // is kDirectI independent chains.  (With the lanes over i and the j's
 // broadcast to them, each 64 pairs took a 16-byte load per lane: 16 cycles of
 // a CU's load path, which bounded the kernel: a step of N = 2,048, 4,096,
-// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 10.0, 15.2,
-// 32.0 and 53.)  It is bound by vector issue, 16 instructions per 64 pairs,
+// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 9.0, 14.0,
+// 30.1 and 52.)  It is bound by vector issue, 16 instructions per 64 pairs,
 // at the large end (11,000: 70% of the issue rate) and by the chain of loads,
 // step, contact terms and sums at the small end.  A wavefront's j are of one
 // material (the wavefronts are divided between the iron and the silicate j),
@@ -1211,6 +1211,18 @@ __device__ __forceinline__ float rows_sum_xyz(float x, float y, float z) {
     return __uint_as_float(u[0]) + __uint_as_float(u[1]);
 }
 
+// x summed over the lanes 8 p + k of each k, on every lane.
+__device__ __forceinline__ float eighths_sum(float x) {
+    x += lane_dpp<0x128>(x);
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+
+// Four float4 records in one load.
+typedef float Float16 __attribute__((ext_vector_type(16), aligned(16)));
+
 template <int MOVE, int W>
 __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel,
@@ -1227,39 +1239,60 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     __shared__ float4 term[W][64];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // W = 16: the arguments in one load, not each where it is first needed.
+    // (Behind this the compiler also loads the records below into vector
+    // registers: see there.)
+    if constexpr (W == 16)
+        asm volatile("" ::"s"(pos), "s"(vel), "s"(blocks), "s"(per_log2), "s"(sims), "s"(force));
     const DirectBlock blk = blocks[blockIdx.x >> per_log2];
     const int i0 = blk.i0 + IB * (blockIdx.x & ((1u << per_log2) - 1u));
     const int start = blk.start, fe_end = blk.fe_end, end = blk.end;
     const SimDesc& sd = sims[blk.sim];
     if (i0 >= end) return;
-    float xi[IB], yi[IB], zi[IB];
-#pragma unroll
-    for (int k = 0; k < IB; ++k) {
-        const float4 p = pos[min(i0 + k, end - 1)];
-        xi[k] = p.x;
-        yi[k] = p.y;
-        zi[k] = p.z;
-    }
     // the wavefronts that take iron j: their share of the 64-blocks
-    const int bf = (fe_end - start + 63) >> 6, bs = (end - fe_end + 63) >> 6;
-    const int wf = bf == 0 ? 0 : bs == 0 ? W : min(max((2 * W * bf + bf + bs) / (2 * (bf + bs)), 1), W - 1);
+    const int wf = blk.iron_waves;
     const bool jfe = wv < wf;
     const int je = jfe ? fe_end : end;
     const int stride = 64 * (jfe ? wf : W - wf);
     int jb = jfe ? start + 64 * wv : fe_end + 64 * (wv - wf);  // the step's 64-block
-
+    float4 nx = pos[min(jb + lane, end - 1)];
+    // Of every workgroup but a simulation's last, one run of records in two
+    // scalar loads, or with W = 16 (where the registers are to spare, and a
+    // vector operand issues in half the cycles of a scalar one) eight vector
+    // loads: eight scalar loads queue behind those of the CU's other
+    // wavefronts, and the last of 16 had its records 1.5 us after the first.
+    // N = 2,048: 7.4 us a call, 6.7 so; 4,096: 12.4 and 11.4; 11,000: 50.7
+    // and 49.2, with nothing divided and the results' operands asked for
+    // before the barrier (the last two 0.2 us).
+    float xi[IB], yi[IB], zi[IB];
+    if (i0 + IB <= end) {
+        const Float16* __restrict__ run = reinterpret_cast<const Float16*>(pos + i0);
+        const Float16 a = run[0], b = run[1];
+#pragma unroll
+        for (int k = 0; k < IB; ++k) {
+            xi[k] = k < 4 ? a[4 * (k & 3)] : b[4 * (k & 3)];
+            yi[k] = k < 4 ? a[4 * (k & 3) + 1] : b[4 * (k & 3) + 1];
+            zi[k] = k < 4 ? a[4 * (k & 3) + 2] : b[4 * (k & 3) + 2];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < IB; ++k) {
+            const float4 p = pos[min(i0 + k, end - 1)];
+            xi[k] = p.x;
+            yi[k] = p.y;
+            zi[k] = p.z;
+        }
+    }
     float ax[IB], ay[IB], az[IB];
 #pragma unroll
     for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
-    CompSum cx, cy, cz;  // lane k: the contact terms of i k
+    CompSum cx, cy, cz;  // lane 8 p + k: the contact terms of i k
     cx.zero();
     cy.zero();
     cz.zero();
     int listed = 0;
-    const int steps = je <= jb ? 0 : (je - jb + stride - 1) / stride;
-    float4 nx = pos[min(jb + lane, end - 1)];
-    for (int st = 0;;) {
-        for (; st < steps && listed <= kWorkOff; ++st) {
+    for (;;) {
+        while (jb < je && listed <= kWorkOff) {
             float4 pj = nx;
             const int j0 = jb;
             jb += stride;
@@ -1300,54 +1333,57 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
         // The listed pairs: the exact contact term minus the gravity term
         // s dp the sums took for it (k_finish's test and arithmetic), a pair
         // per lane, then added per i in list order.
-                    // the law read here: hoisted out, its registers spill the loop's
-                    const SimDesc* lp = sims + blk.sim;
-                    asm volatile("" : "+s"(lp));
-                    const PairLaw& law = lp->law;
-                    for (int e0 = 0; e0 < listed; e0 += 64) {
-                        const int cnt = min(64, listed - e0);
-                        wave_lds_sync();
-                        float4 t = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
-                        if (lane < cnt) {
-                            const int e = list[wv][e0 + lane];
-                            const int k = e >> 24, jj = e & 0xffffff;
-                            const float4 pi = pos[i0 + k], pj = pos[jj];
-                            const float4 vi = vel[i0 + k], vj = vel[jj];
-                            const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-                            const float r2 = dx * dx + dy * dy + dz * dz;
-                            const float r = sqrtf(r2);
-                            if (r < 1.0f) {
-                                const float invr = 1.0f / r;
-                                const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
-                                const float dot = dx * dvx + dy * dvy + dz * dvz;
-                                const int test = (int)(i0 + k < fe_end) + (int)jfe;
-                                const float fm = contact_pair_mag(law, test, r, r2, dot);
-                                const float sf = gravity_product(law, test) * fast_inv_r3(fast_r2(dx, dy, dz));
-                                t = make_float4(fm * dx * invr - sf * dx, fm * dy * invr - sf * dy, fm * dz * invr - sf * dz,
-                                                __int_as_float(k));
-                            }
-                        }
-                        term[wv][lane] = t;
-                        wave_lds_sync();
-                        // a batch's terms of one i: a handful, in a plain float sum
-                        float bx = 0.0f, by = 0.0f, bz = 0.0f;
-                        for (int q = 0; q < cnt; q += 4) {
-                            float4 u[4];
-        #pragma unroll
-                            for (int w = 0; w < 4; ++w) u[w] = term[wv][q + w];
-        #pragma unroll
-                            for (int w = 0; w < 4; ++w) {
-                                const bool mine = __float_as_int(u[w].w) == lane;
-                                bx += mine ? u[w].x : 0.0f;
-                                by += mine ? u[w].y : 0.0f;
-                                bz += mine ? u[w].z : 0.0f;
-                            }
-                        }
-                        cx.add(bx);
-                        cy.add(by);
-                        cz.add(bz);
-                    }
-        if (st >= steps) break;
+        // the law read here: hoisted out, its registers spill the loop's
+        const SimDesc* lp = sims + blk.sim;
+        asm volatile("" : "+s"(lp));
+        const PairLaw& law = lp->law;
+        for (int e0 = 0; e0 < listed; e0 += 64) {
+            const int cnt = min(64, listed - e0);
+            wave_lds_sync();
+            float4 t = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
+            if (lane < cnt) {
+                const int e = list[wv][e0 + lane];
+                const int k = e >> 24, jj = e & 0xffffff;
+                const float4 pi = pos[i0 + k], pj = pos[jj];
+                const float4 vi = vel[i0 + k], vj = vel[jj];
+                const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+                const float r2 = dx * dx + dy * dy + dz * dz;
+                const float r = sqrtf(r2);
+                if (r < 1.0f) {
+                    const float invr = 1.0f / r;
+                    const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+                    const float dot = dx * dvx + dy * dvy + dz * dvz;
+                    const int test = (int)(i0 + k < fe_end) + (int)jfe;
+                    const float fm = contact_pair_mag(law, test, r, r2, dot);
+                    const float sf = gravity_product(law, test) * fast_inv_r3(fast_r2(dx, dy, dz));
+                    t = make_float4(fm * dx * invr - sf * dx, fm * dy * invr - sf * dy, fm * dz * invr - sf * dz,
+                                    __int_as_float(k));
+                }
+            }
+            term[wv][lane] = t;
+            wave_lds_sync();
+            // A batch's terms of one i, a handful, in plain float sums: lane
+            // 8 p + k adds those of i k among every eighth term, then the
+            // eight lanes of an i are added (a lane per i over all 64 terms
+            // took 1 us a batch: a step of N = 1,024 in contact 10.1 us, 8.1
+            // so, of 8,192 33.3 and 30.6).
+            float bx = 0.0f, by = 0.0f, bz = 0.0f;
+#pragma unroll 4
+            for (int u = 0; u < 8; ++u) {
+                const float4 o = term[wv][8 * u + (lane >> 3)];
+                const bool mine = __float_as_int(o.w) == (lane & 7);
+                bx += mine ? o.x : 0.0f;
+                by += mine ? o.y : 0.0f;
+                bz += mine ? o.z : 0.0f;
+            }
+            bx = eighths_sum(bx);
+            by = eighths_sum(by);
+            bz = eighths_sum(bz);
+            cx.add(bx);
+            cy.add(by);
+            cz.add(bz);
+        }
+        if (jb >= je) break;
         listed = 0;
     }
     grav[wv][lane] = rows_sum_xyz(row_sums8(ax, lane & 15), row_sums8(ay, lane & 15), row_sums8(az, lane & 15));
@@ -1359,19 +1395,30 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
         contact[wv][4][lane] = cz.s;
         contact[wv][5][lane] = cz.c;
     }
-    __syncthreads();
     // Wavefront c < 3 adds component c: lane q * 8 + k takes the sums of i k
     // of wavefronts q and q + 8, then the eight lanes of an i are added.  The
-    // move's components are independent; wavefront 3 carries .w over.
-    if (wv > 3) return;
+    // move's components are independent; wavefront 3 carries .w over.  What
+    // this reads is asked for before the others are waited for.
     const int k = lane & 7, q = lane >> 3;
     const int i = i0 + k;
-    const bool ife = i < fe_end;
+    float g[W / 8] = {}, v = 0.0f, p = 0.0f;
+    if (wv < 3) {
+#pragma unroll
+        for (int u = 0; u < W / 8; ++u)
+            g[u] = gravity_product(sd.law, (int)(i < fe_end) + (int)(q + 8 * u < wf));
+    }
+    if constexpr (MOVE != 0)
+        if (wv < 4 && i < end) {
+            v = reinterpret_cast<const float*>(vel + i)[wv];
+            p = reinterpret_cast<const float*>(pos + i)[wv];
+        }
+    __syncthreads();
+    if (wv > 3) return;
     if (wv == 3) {
         if constexpr (MOVE != 0)
             if (lane < IB && i < end) {
-                mv.pout[i].w = pos[i].w;
-                mv.vout[i].w = vel[i].w;
+                mv.pout[i].w = p;
+                mv.vout[i].w = v;
             }
         return;
     }
@@ -1380,7 +1427,7 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
 #pragma unroll
     for (int u = 0; u < W / 8; ++u) {
         const int w = q + 8 * u;
-        t.add_product(gravity_product(sd.law, (int)ife + (int)(w < wf)), grav[w][16 * wv + k]);
+        t.add_product(g[u], grav[w][16 * wv + k]);
         t.add(contact[w][2 * wv][k]);
         t.c += contact[w][2 * wv + 1][k];
     }
@@ -1411,8 +1458,6 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
             temp = mv.dt_over_mass_fe;
             damp = mv.damp1;
         }
-        float v = reinterpret_cast<const float*>(vel + i)[wv];
-        float p = reinterpret_cast<const float*>(pos + i)[wv];
         if constexpr (MOVE == 1)
             v += f * temp;
         else
