@@ -1286,7 +1286,7 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     float ax[IB], ay[IB], az[IB];
 #pragma unroll
     for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
-    CompSum cx, cy, cz;  // lane 8 p + k: the contact terms of i k
+    CompSum cx, cy, cz;  // lane k: the contact terms of i k
     cx.zero();
     cy.zero();
     cz.zero();
@@ -1362,23 +1362,50 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
             }
             term[wv][lane] = t;
             wave_lds_sync();
-            // A batch's terms of one i, a handful, in plain float sums: lane
-            // 8 p + k adds those of i k among every eighth term, then the
-            // eight lanes of an i are added (a lane per i over all 64 terms
-            // took 1 us a batch: a step of N = 1,024 in contact 10.1 us, 8.1
-            // so, of 8,192 33.3 and 30.6).
+            // A batch's terms of one i, a handful, in a plain float sum: with
+            // W = 16 lane k takes those of i k in list order, four loads in
+            // flight; with W = 8, where that form's scalar registers spill,
+            // lane 8 p + k takes those of i k among every eighth term, and the
+            // eight lanes of an i are added.  (All 64 terms looked at by each
+            // of eight lanes took 1 us a batch: a step of N = 1,024 in
+            // contact 10.1 us, 8.1 so, of 8,192 33.5 and 30.6.)
             float bx = 0.0f, by = 0.0f, bz = 0.0f;
+            if constexpr (W == 16) {
+                unsigned long long m = 0;
+#pragma unroll
+                for (int k = 0; k < IB; ++k) {
+                    const unsigned long long of_k = __ballot(__float_as_int(t.w) == k);
+                    m = lane == k ? of_k : m;
+                }
+                while (m) {
+                    float4 u[4];
+                    bool on[4];
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        on[w] = m != 0;
+                        u[w] = term[wv][on[w] ? __builtin_ctzll(m) : 0];
+                        m &= m - 1;
+                    }
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        bx += on[w] ? u[w].x : 0.0f;
+                        by += on[w] ? u[w].y : 0.0f;
+                        bz += on[w] ? u[w].z : 0.0f;
+                    }
+                }
+            } else {
 #pragma unroll 4
-            for (int u = 0; u < 8; ++u) {
-                const float4 o = term[wv][8 * u + (lane >> 3)];
-                const bool mine = __float_as_int(o.w) == (lane & 7);
-                bx += mine ? o.x : 0.0f;
-                by += mine ? o.y : 0.0f;
-                bz += mine ? o.z : 0.0f;
+                for (int u = 0; u < 8; ++u) {
+                    const float4 o = term[wv][8 * u + (lane >> 3)];
+                    const bool mine = __float_as_int(o.w) == (lane & 7);
+                    bx += mine ? o.x : 0.0f;
+                    by += mine ? o.y : 0.0f;
+                    bz += mine ? o.z : 0.0f;
+                }
+                bx = eighths_sum(bx);
+                by = eighths_sum(by);
+                bz = eighths_sum(bz);
             }
-            bx = eighths_sum(bx);
-            by = eighths_sum(by);
-            bz = eighths_sum(bz);
             cx.add(bx);
             cy.add(by);
             cz.add(bz);
