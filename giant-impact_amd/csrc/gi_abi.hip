@@ -588,15 +588,6 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
     return 0;
 }
 
-// Wavefronts per workgroup of k_direct for n particles (of all simulations):
-// up to 2,048 particles there is a workgroup per CU at most, and 16
-// wavefronts shorten its chain (a step of N = 2,048 takes 9.8 us against 10.2
-// with 8); above, 8 leave room for the next workgroup beside the running ones
-// (N = 3,000 13.1 against 15.4 us, 4,096 15.2 against 17.9, 11,000 53 against
-// 69; four wavefronts were slower up to 8,192 and even above).
-constexpr long long kDirectWideMaxN = 2048;
-static int direct_waves(long long n) { return n <= kDirectWideMaxN ? 16 : 8; }
-
 // The plan of one force evaluation over `sims`: the mutual pass's tasks and
 // rows for the simulations that take it, then the one-sided pass's chunks
 // and tasks for the rest, the contact-grid bucket ranges and the moment
@@ -643,7 +634,7 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
                 for (int i0 = sims[si].start; i0 < sims[si].end; i0 += ib)
                     p.dblocks.push_back(DirectBlock{(int)si, i0, sims[si].start, sims[si].fe_end, sims[si].end,
                                                     direct_iron_waves(sims[si].start, sims[si].fe_end, sims[si].end,
-                                                                      direct_waves(ntot)),
+                                                                      kDirectForceWaves),
                                                     0, 0});
         p.direct = true;
     }
@@ -1145,15 +1136,12 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
 
 // k_direct over a block table of 64 / lanes i-particles per entry.
 template <int MOVE>
-static void direct_kernel(int lanes, int waves, int nblocks, hipStream_t st, const float4* pos, const float4* vel,
+static void direct_kernel(int lanes, int nblocks, hipStream_t st, const float4* pos, const float4* vel,
                           const DirectBlock* blocks, const SimDesc* sims, float4* force, const FusedMove& mv) {
     int per_log2 = 0;
     while ((kDirectI << per_log2) * lanes < 64) ++per_log2;
-    const dim3 grid((unsigned)nblocks << per_log2), block(64 * waves);
-    if (waves == 16)
-        hipLaunchKernelGGL((k_direct<MOVE, 16>), grid, block, 0, st, pos, vel, blocks, per_log2, sims, force, mv);
-    else
-        hipLaunchKernelGGL((k_direct<MOVE, 8>), grid, block, 0, st, pos, vel, blocks, per_log2, sims, force, mv);
+    hipLaunchKernelGGL(k_direct<MOVE>, dim3((unsigned)nblocks << per_log2), dim3(64 * kDirectForceWaves), 0, st, pos,
+                       vel, blocks, per_log2, sims, force, mv);
 }
 
 // The direct pass of the current plan: the force, or with pot the
@@ -1171,7 +1159,7 @@ static int launch_direct(DevCtx* ctx, Workspace* ws, const float4* pos, const fl
         GI_HIP(hipEventRecord(t2.a, st));
         GI_HIP(hipEventRecord(t0.a, st));
     }
-    const int lanes = p.direct_lanes, waves = direct_waves(p.ntot);
+    const int lanes = p.direct_lanes;
     const DirectBlock* bl = ws->dblocks.p;
     if (pot) {
         const dim3 grid(nb), block(64 * kDirectWaves);
@@ -1184,11 +1172,11 @@ static int launch_direct(DevCtx* ctx, Workspace* ws, const float4* pos, const fl
         else
             hipLaunchKernelGGL(k_direct_potential<1>, grid, block, 0, st, pos, bl, ws->sims.p, ws->pe.p);
     } else if (move == 1) {
-        direct_kernel<1>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+        direct_kernel<1>(lanes, nb, st, pos, vel, bl, ws->sims.p, force, mv);
     } else if (move == 2) {
-        direct_kernel<2>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+        direct_kernel<2>(lanes, nb, st, pos, vel, bl, ws->sims.p, force, mv);
     } else {
-        direct_kernel<0>(lanes, waves, nb, st, pos, vel, bl, ws->sims.p, force, mv);
+        direct_kernel<0>(lanes, nb, st, pos, vel, bl, ws->sims.p, force, mv);
     }
     GI_HIP(hipGetLastError());
     if (timed) {
@@ -1844,8 +1832,8 @@ int gi_force_collision_noalloc(const gi_float4* pos, const gi_float4* vel, gi_fl
                          kNoAllocMaxBlocks);
     hipStream_t st = as_stream(stream);
     hipLaunchKernelGGL(k_noalloc_plan, dim3(nblk(nb, 256)), dim3(256), 0, st, sp, make_sim(0, c->NFe, n, law_of(c)),
-                       nb, ib, direct_iron_waves(0, c->NFe, n, direct_waves(n)));
-    direct_kernel<0>(lanes, direct_waves(n), nb, st, (const float4*)pos, (const float4*)vel, sp->blocks, &sp->sim,
+                       nb, ib, direct_iron_waves(0, c->NFe, n, kDirectForceWaves));
+    direct_kernel<0>(lanes, nb, st, (const float4*)pos, (const float4*)vel, sp->blocks, &sp->sim,
                      (float4*)force, FusedMove{});
     GI_HIP(hipGetLastError());
     return 0;

@@ -1146,8 +1146,8 @@ __global__ __launch_bounds__(64 * kContactWaves) void k_contact_corr(int ntot, c
 // is kDirectI independent chains.  (With the lanes over i and the j's
 // broadcast to them, each 64 pairs took a 16-byte load per lane: 16 cycles of
 // a CU's load path, which bounded the kernel: a step of N = 2,048, 4,096,
-// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 9.0, 14.0,
-// 30.1 and 52.)  It is bound by vector issue, 16 instructions per 64 pairs,
+// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 8.0, 12.6,
+// 29.1 and 51.)  It is bound by vector issue, 16 instructions per 64 pairs,
 // at the large end (11,000: 70% of the issue rate) and by the chain of loads,
 // step, contact terms and sums at the small end.  A wavefront's j are of one
 // material (the wavefronts are divided between the iron and the silicate j),
@@ -1160,8 +1160,14 @@ __global__ __launch_bounds__(64 * kContactWaves) void k_contact_corr(int ntot, c
 // lane: the exact contact term minus the gravity term, with the arithmetic of
 // k_finish, added per i in list order in a compensated sum.  The wavefronts'
 // sums are added in a compensated float sum in a fixed order, so the result
-// depends on the simulation and the number of wavefronts alone.
+// depends on the simulation alone.
+//
+// Eight wavefronts per workgroup, so that another has room beside the running
+// ones: a call takes 5.4, 6.6, 9.6 and 18.0 us at N = 1,024, 2,048, 3,072 and
+// 6,000, with 16 wavefronts 5.8, 6.7, 11.7 and 23.5 (four were slower up to
+// 8,192 and even above).
 constexpr int kDirectI = 8;
+constexpr int kDirectForceWaves = 8;
 // r^2 (with FMAs and kSelfEps) of every pair whose exactly rounded r is below
 // 1 lies below this: the margin covers the few ulps between the two forms.
 constexpr float kDirectContactR2 = 1.0001f;
@@ -1223,13 +1229,14 @@ __device__ __forceinline__ float eighths_sum(float x) {
 // Four float4 records in one load.
 typedef float Float16 __attribute__((ext_vector_type(16), aligned(16)));
 
-template <int MOVE, int W>
-__global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ pos,
+template <int MOVE>
+__global__ __launch_bounds__(64 * kDirectForceWaves) void k_direct(const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel,
                                                    const DirectBlock* __restrict__ blocks, int per_log2,
                                                    const SimDesc* __restrict__ sims, float4* __restrict__ force,
                                                    FusedMove mv) {
-    static_assert(W == 8 || W == 16, "wavefronts per workgroup");
+    constexpr int W = kDirectForceWaves;
+    static_assert(W == 8, "a wavefront's eight lanes per particle add the wavefronts' sums");
     constexpr int IB = kDirectI;
     constexpr int kWorkOff = 128;             // listed pairs that are worked off before the next step
     constexpr int kList = kWorkOff + 64 * IB;  // and what one step can add
@@ -1239,11 +1246,6 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     __shared__ float4 term[W][64];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // W = 16: the arguments in one load, not each where it is first needed.
-    // (Behind this the compiler also loads the records below into vector
-    // registers: see there.)
-    if constexpr (W == 16)
-        asm volatile("" ::"s"(pos), "s"(vel), "s"(blocks), "s"(per_log2), "s"(sims), "s"(force));
     const DirectBlock blk = blocks[blockIdx.x >> per_log2];
     const int i0 = blk.i0 + IB * (blockIdx.x & ((1u << per_log2) - 1u));
     const int start = blk.start, fe_end = blk.fe_end, end = blk.end;
@@ -1257,13 +1259,9 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     int jb = jfe ? start + 64 * wv : fe_end + 64 * (wv - wf);  // the step's 64-block
     float4 nx = pos[min(jb + lane, end - 1)];
     // Of every workgroup but a simulation's last, one run of records in two
-    // scalar loads, or with W = 16 (where the registers are to spare, and a
-    // vector operand issues in half the cycles of a scalar one) eight vector
-    // loads: eight scalar loads queue behind those of the CU's other
-    // wavefronts, and the last of 16 had its records 1.5 us after the first.
-    // N = 2,048: 7.4 us a call, 6.7 so; 4,096: 12.4 and 11.4; 11,000: 50.7
-    // and 49.2, with nothing divided and the results' operands asked for
-    // before the barrier (the last two 0.2 us).
+    // scalar loads: eight queue behind those of the CU's other wavefronts.
+    // N = 4,096: 12.4 us a call, 11.4 so; 11,000: 50.7 and 49.2, with nothing
+    // divided and the results' operands asked for before the barrier.
     float xi[IB], yi[IB], zi[IB];
     if (i0 + IB <= end) {
         const Float16* __restrict__ run = reinterpret_cast<const Float16*>(pos + i0);
@@ -1286,7 +1284,7 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     float ax[IB], ay[IB], az[IB];
 #pragma unroll
     for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
-    CompSum cx, cy, cz;  // lane k: the contact terms of i k
+    CompSum cx, cy, cz;  // lane 8 p + k: the contact terms of i k
     cx.zero();
     cy.zero();
     cz.zero();
@@ -1362,50 +1360,23 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
             }
             term[wv][lane] = t;
             wave_lds_sync();
-            // A batch's terms of one i, a handful, in a plain float sum: with
-            // W = 16 lane k takes those of i k in list order, four loads in
-            // flight; with W = 8, where that form's scalar registers spill,
-            // lane 8 p + k takes those of i k among every eighth term, and the
+            // A batch's terms of one i, a handful, in plain float sums: lane
+            // 8 p + k takes those of i k among every eighth term, then the
             // eight lanes of an i are added.  (All 64 terms looked at by each
             // of eight lanes took 1 us a batch: a step of N = 1,024 in
-            // contact 10.1 us, 8.1 so, of 8,192 33.5 and 30.6.)
+            // contact 9.3 us, 7.0 so, of 8,192 33.5 and 29.6.)
             float bx = 0.0f, by = 0.0f, bz = 0.0f;
-            if constexpr (W == 16) {
-                unsigned long long m = 0;
-#pragma unroll
-                for (int k = 0; k < IB; ++k) {
-                    const unsigned long long of_k = __ballot(__float_as_int(t.w) == k);
-                    m = lane == k ? of_k : m;
-                }
-                while (m) {
-                    float4 u[4];
-                    bool on[4];
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        on[w] = m != 0;
-                        u[w] = term[wv][on[w] ? __builtin_ctzll(m) : 0];
-                        m &= m - 1;
-                    }
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        bx += on[w] ? u[w].x : 0.0f;
-                        by += on[w] ? u[w].y : 0.0f;
-                        bz += on[w] ? u[w].z : 0.0f;
-                    }
-                }
-            } else {
 #pragma unroll 4
-                for (int u = 0; u < 8; ++u) {
-                    const float4 o = term[wv][8 * u + (lane >> 3)];
-                    const bool mine = __float_as_int(o.w) == (lane & 7);
-                    bx += mine ? o.x : 0.0f;
-                    by += mine ? o.y : 0.0f;
-                    bz += mine ? o.z : 0.0f;
-                }
-                bx = eighths_sum(bx);
-                by = eighths_sum(by);
-                bz = eighths_sum(bz);
+            for (int u = 0; u < 8; ++u) {
+                const float4 o = term[wv][8 * u + (lane >> 3)];
+                const bool mine = __float_as_int(o.w) == (lane & 7);
+                bx += mine ? o.x : 0.0f;
+                by += mine ? o.y : 0.0f;
+                bz += mine ? o.z : 0.0f;
             }
+            bx = eighths_sum(bx);
+            by = eighths_sum(by);
+            bz = eighths_sum(bz);
             cx.add(bx);
             cy.add(by);
             cz.add(bz);
@@ -1422,18 +1393,14 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
         contact[wv][4][lane] = cz.s;
         contact[wv][5][lane] = cz.c;
     }
-    // Wavefront c < 3 adds component c: lane q * 8 + k takes the sums of i k
-    // of wavefronts q and q + 8, then the eight lanes of an i are added.  The
-    // move's components are independent; wavefront 3 carries .w over.  What
-    // this reads is asked for before the others are waited for.
-    const int k = lane & 7, q = lane >> 3;
+    // Wavefront c < 3 adds component c: lane w * 8 + k takes the sums of i k
+    // of wavefront w, then the eight lanes of an i are added.  The move's
+    // components are independent; wavefront 3 carries .w over.  What this
+    // reads is asked for before the others are waited for.
+    const int k = lane & 7, w = lane >> 3;
     const int i = i0 + k;
-    float g[W / 8] = {}, v = 0.0f, p = 0.0f;
-    if (wv < 3) {
-#pragma unroll
-        for (int u = 0; u < W / 8; ++u)
-            g[u] = gravity_product(sd.law, (int)(i < fe_end) + (int)(q + 8 * u < wf));
-    }
+    float g = 0.0f, v = 0.0f, p = 0.0f;
+    if (wv < 3) g = gravity_product(sd.law, (int)(i < fe_end) + (int)(w < wf));
     if constexpr (MOVE != 0)
         if (wv < 4 && i < end) {
             v = reinterpret_cast<const float*>(vel + i)[wv];
@@ -1451,13 +1418,9 @@ __global__ __launch_bounds__(64 * W) void k_direct(const float4* __restrict__ po
     }
     CompSum t;
     t.zero();
-#pragma unroll
-    for (int u = 0; u < W / 8; ++u) {
-        const int w = q + 8 * u;
-        t.add_product(g[u], grav[w][16 * wv + k]);
-        t.add(contact[w][2 * wv][k]);
-        t.c += contact[w][2 * wv + 1][k];
-    }
+    t.add_product(g, grav[w][16 * wv + k]);
+    t.add(contact[w][2 * wv][k]);
+    t.c += contact[w][2 * wv + 1][k];
 #pragma unroll
     for (int m = 8; m < 64; m <<= 1) {
         CompSum o;
@@ -2282,15 +2245,12 @@ GI_GRAVITY_INST(8, true, 0)
 #undef GI_GRAVITY_INST
 #define GI_MUTUAL_INST(R, POT) \
     template __global__ void k_mutual<R, POT>(const float4*, const MutualTask*, int, const SimDesc*, float*, float*);
-#define GI_DIRECT_INST(MOVE, W)                                                                            \
-    template __global__ void k_direct<MOVE, W>(const float4*, const float4*, const DirectBlock*, int,      \
-                                               const SimDesc*, float4*, FusedMove);
-GI_DIRECT_INST(0, 8)
-GI_DIRECT_INST(1, 8)
-GI_DIRECT_INST(2, 8)
-GI_DIRECT_INST(0, 16)
-GI_DIRECT_INST(1, 16)
-GI_DIRECT_INST(2, 16)
+#define GI_DIRECT_INST(MOVE)                                                                                     \
+    template __global__ void k_direct<MOVE>(const float4*, const float4*, const DirectBlock*, int, const SimDesc*, \
+                                            float4*, FusedMove);
+GI_DIRECT_INST(0)
+GI_DIRECT_INST(1)
+GI_DIRECT_INST(2)
 #undef GI_DIRECT_INST
 #define GI_DIRECT_POT_INST(S) \
     template __global__ void k_direct_potential<S>(const float4*, const DirectBlock*, const SimDesc*, double*);
