@@ -1885,10 +1885,11 @@ __global__ void k_recenter_apply(float4* __restrict__ pos, float4* __restrict__ 
 // is looked up by it (0.24 us a group or run instead of 0.28), and the
 // groups' own joins, 11 us in the chains' seven workgroups, run side by side.
 // Bound by the join's chain of dependent FP64 operations.  The impact states
-// need 0 to 14 of 1,024 runs step by step.  N = 65,536: 105 us a call (sums
-// 5 us, bounds 17, runs 28, join 45 to 77, apply 5; 122 us with the groups
-// joined in the chains' own workgroups and one start tried) against 3,404
-// step by step; windows of 128 took 135.
+// need 0 to 14 of 1,024 runs of a chain step by step.  N = 65,536, eight
+// impact states: 98 to 172 us a call, 119 on average (sums 5 us, bounds 17,
+// runs 28, join 35 to 110, apply 5; 106 to 191 and 137 with the groups joined
+// in the chains' own workgroups and one start tried) against 3,404 step by
+// step; windows of 128 took 10% longer.
 constexpr int kRcChains = 7;
 constexpr int kRcStarts = 16;
 constexpr int kRcGroup = 16;     // runs per group

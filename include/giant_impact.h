@@ -353,8 +353,8 @@ int gi_find_earth_moon(const gi_float4 *pos, const gi_float4 *vel, int n, int nf
  * lane (1, 2, 4 or 8), variant = the all-pairs pass (0: one-sided, r^-3 as rsq
  * cubed; 1: one-sided, rsq*rcp; 2: mutual -- each pair evaluated once for both
  * particles, rows of 64*r particles; 3: direct -- small simulations, the whole
- * force, contacts included, in one launch, r = lanes per i-particle: 1, 2,
- * 4 or 8),
+ * force, contacts included, in one launch, r = 1, 2, 4 or 8: 64 / r
+ * i-particles per entry of the block table),
  * chunk_len = j-particles per task (0 =
  * derived from target_tasks),
  * target_tasks = wavefront tasks to aim for, min_chunk = lower bound of
@@ -407,7 +407,7 @@ int gi_set_dispatch_limit(long long max_tasks);
 int gi_set_contact_overlap(int enable);
 
 /* Contact walk (lanes = 0, the default: nine lanes per particle for force
- * evaluations of up to 49,152 particles, one lane per particle above): the
+ * evaluations of up to 49,152^2 pairs, one lane per particle above): the
  * contact corrections' walk over a particle's 27 neighbour cells, forced to
  * one lane per particle (1) or one lane per row of three cells (9).  The two
  * forms share their arithmetic: the corrections are bitwise the same either
