@@ -1882,14 +1882,16 @@ __global__ void k_recenter_apply(float4* __restrict__ pos, float4* __restrict__ 
 // Joining looks at all 16 starts at once, one per lane of a row, and takes the
 // first that holds: 24 groups of an impact state's 448 go run by run instead
 // of the 27 where only the start picked by the difference was tried, nothing
-// is looked up by it (0.24 us a group or run instead of 0.28), and the
-// groups' own joins, 11 us in the chains' seven workgroups, run side by side.
+// is looked up by it, and the groups' own joins, 11 us in the chains' seven
+// workgroups, run side by side.  What it compares is worked out beforehand, a
+// candidate per lane (0.24 us a group or run before).
 // Bound by the join's chain of dependent FP64 operations.  The impact states
 // need 0 to 14 of 1,024 runs of a chain step by step.  N = 65,536, eight
-// impact states: 98 to 172 us a call, 119 on average (sums 5 us, bounds 17,
-// runs 28, join 35 to 110, apply 5; 106 to 191 and 137 with the groups joined
-// in the chains' own workgroups and one start tried) against 3,404 step by
-// step; windows of 128 took 10% longer.
+// impact states: 75 to 140 us a call, 93 on average (sums 5 us, bounds 16,
+// runs 17, join 25 to 95, apply 5; 119 with an element per load of all 16
+// lanes and the candidates worked out as they are met, 137 with the groups
+// joined in the chains' own workgroups and one start tried) against 3,404
+// step by step; windows of 128 took 10% longer.
 constexpr int kRcChains = 7;
 constexpr int kRcStarts = 16;
 constexpr int kRcGroup = 16;     // runs per group
@@ -1975,9 +1977,17 @@ __global__ __launch_bounds__(64 * kRcWindowWaves) void k_rc_bounds(const float4*
     if (w >= wk.nwin) return;
     // the prefix before the window
     double p[kRcChains] = {};
-    for (int k = lane; k < w; k += 64)
+    for (int k = lane; k < w; k += 64 * 4) {
+        double v[4][kRcChains];  // four round trips to memory in one
 #pragma unroll
-        for (int c = 0; c < kRcChains; ++c) p[c] += wk.sums[c * wk.nwin + k];
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < kRcChains; ++c) v[u][c] = wk.sums[c * wk.nwin + min(k + 64 * u, w - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < kRcChains; ++c) p[c] += k + 64 * u < w ? v[u][c] : 0.0;
+    }
     // this lane's share of the window: consecutive elements
     const int per = wk.window / 64;
     const int end = rc_window_end(wk, w, n);
@@ -2058,10 +2068,10 @@ __device__ __forceinline__ double rc_ulp(float g) {
 }
 __device__ __forceinline__ float rc_start(float g, int j) { return (float)((double)g + (double)j * rc_ulp(g)); }
 
-// One step with term t = x * mass: the sum's rounding to float, its binade
+// One step with term t: the sum's rounding to float, its binade
 // and its distance from the binade's ends, rounded down to the sum's 21
 // leading bits.  A zero term changes nothing from any start.
-__device__ __forceinline__ void rc_step(float& a, float x, double t, int& binade, float& room) {
+__device__ __forceinline__ void rc_step(float& a, double t, int& binade, float& room) {
     const double s = (double)a + t;
     const int hi = __double2hiint(s) & 0x7fffffff;
     const int e = hi >> 20;
@@ -2069,22 +2079,36 @@ __device__ __forceinline__ void rc_step(float& a, float x, double t, int& binade
     float r = __builtin_amdgcn_ldexpf((float)min(m, 0xfffff - m), e - 1023 - 20);
     // well inside the float range only (not infinite or NaN)
     if ((unsigned)(e - (1023 - 80)) > 160u) r = -1.0f;
-    if (x != 0.0f) {
+    if (t != 0.0) {
         binade = max(binade, e);
         room = fminf(room, r);
     }
     a = (float)s;
 }
 
-// Whether run (or group) r, taken from `start`, holds for the true start a,
-// and the difference d of the two.
-__device__ __forceinline__ bool rc_holds(float a, float start, const RcRun& r, double& d) {
-    d = (double)a - (double)start;
-    const double k = __builtin_amdgcn_ldexp(d, 1023 + 22 - r.binade);  // in pairs of ulps of the run's largest binade
-    const bool exact = (double)a - d == (double)start;
-    const bool shift = fabs(d) < (double)r.room && k == rint(k);
-    // binade 0: every term is zero
-    return exact && (d == 0.0 || r.binade == 0 || shift) && r.binade >= 0;
+// A run (or group) from one start as a join asks for it, worked out beforehand
+// in FP64.  A group that does not hold starts at NaN; one whose terms are all
+// zero takes any shift.
+struct RcCand {
+    double start, end, room, pairs;  // pairs: shifts in pairs of ulps of the largest binade, over the shift
+};
+__device__ __forceinline__ RcCand rc_cand(const RcRun& r, float start) {
+    RcCand q{(double)start, (double)r.end, (double)r.room, __builtin_amdgcn_ldexp(1.0, 1023 + 22 - r.binade)};
+    if (r.binade == 0) {
+        q.room = __builtin_inf();
+        q.pairs = 0.0;
+    } else if (r.binade < 0) {
+        q.start = __builtin_nan("");
+    }
+    return q;
+}
+// Whether it holds for the true start a, a float, and the difference d of the
+// two starts: then a's end is the float q.end + d.
+__device__ __forceinline__ bool rc_holds(double a, const RcCand& q, double& d) {
+    d = a - q.start;
+    const double k = d * q.pairs;
+    const bool shift = (fabs(d) < q.room) & (k == rint(k));
+    return (a - d == q.start) & (shift | (d == 0.0));
 }
 
 // Lane j of a row of 16 holds a run's (or group's) start j and what it led
@@ -2095,13 +2119,26 @@ __device__ __forceinline__ int rc_pick(bool holds, int lane) {
     return m ? (lane & 48) + __builtin_ctz(m) : -1;
 }
 
+// Sixteen steps from U on, step u with lane u's term of each row of 16 lanes.
+template <int U = 0>
+__device__ __forceinline__ void rc_steps16(RcRun& r, double t) {
+    if constexpr (U < 16) {
+        rc_step(r.end,
+                __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(t), 0x150 + U, 0xF, 0xF, true),
+                                 __builtin_amdgcn_mov_dpp(__double2loint(t), 0x150 + U, 0xF, 0xF, true)),
+                r.binade, r.room);
+        rc_steps16<U + 1>(r, t);
+    }
+}
+
 // One workgroup per group of a chain: the group's runs from their starts, a
-// run and start per lane, then the runs joined from each of the group's
+// run and start per lane (a run's elements 16 at a time, one load per lane of
+// its row, four such loads in flight), then the runs joined from each of the group's
 // starts, a row of lanes per start.
 __global__ __launch_bounds__(256) void k_rc_runs(const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                  int nfe, double mass_fe, double mass_si, RcWork wk) {
-    __shared__ RcRun run[kRcGroup][kRcStarts];
-    __shared__ float guess[kRcGroup];
+    __shared__ RcCand run[kRcGroup][kRcStarts];
+    __shared__ int binade[kRcGroup][kRcStarts];
     const int c = blockIdx.x / wk.ngroups, g = blockIdx.x % wk.ngroups;
     const int row = threadIdx.x / kRcStarts, j = threadIdx.x % kRcStarts, lane = threadIdx.x & 63;
     const int s0 = g * kRcGroup, ns = min(kRcGroup, wk.nwin - s0);
@@ -2110,82 +2147,87 @@ __global__ __launch_bounds__(256) void k_rc_runs(const float4* __restrict__ pos,
         const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
         const int b = bound[s], e = bound[s + 1];
         const float gs = wk.guess[c * wk.nwin + s];
-        if (j == 0) guess[row] = gs;
         RcRun r{rc_start(gs, j), 0, kRcRoom, 0};
-        float x[8], nx[8];
+        float x[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = rc_value(pos, vel, c, min(b + u, e - 1));
-        for (int k = b; k < e; k += 8) {
+        for (int u = 0; u < 4; ++u) x[u] = rc_value(pos, vel, c, min(b + 16 * u + j, e - 1));
+        for (int k = b; k < e; k += 64) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) nx[u] = rc_value(pos, vel, c, min(k + 8 + u, e - 1));
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (k + u < e) rc_step(r.end, x[u], (double)x[u] * (k + u < nfe ? mass_fe : mass_si), r.binade, r.room);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) x[u] = nx[u];
+            for (int u = 0; u < 4; ++u) {
+                const int i = k + 16 * u + j;
+                // past the run's end: -0 leaves every sum as it is
+                const double t = i < e ? (double)x[u] * (i < nfe ? mass_fe : mass_si) : -0.0;
+                x[u] = rc_value(pos, vel, c, min(i + 64, e - 1));
+                rc_steps16(r, t);
+            }
         }
         wk.runs[((size_t)c * wk.nwin + s) * kRcStarts + j] = r;
-        run[row][j] = r;
+        run[row][j] = rc_cand(r, rc_start(gs, j));
+        binade[row][j] = r.binade;
     }
     __syncthreads();
-    RcRun x{rc_start(guess[0], row), 0, kRcRoom, 0};
+    RcRun x{(float)run[0][row].start, 0, kRcRoom, 0};
     for (int s = 0; s < ns; ++s) {
-        const RcRun r = run[s][j];
+        const RcCand q = run[s][j];
         double d;
-        const int at = rc_pick(rc_holds(x.end, rc_start(guess[s], j), r, d), lane);
+        const int at = rc_pick(rc_holds((double)x.end, q, d), lane);
         const int from = max(at, 0);
         // rounded down: the least factor below 1 takes more than the
         // subtraction's and the conversion's rounding
-        const float room = (float)(((double)r.room - fabs(d)) * (1.0 - 0x1p-20));
-        x.end = __shfl((float)((double)r.end + d), from);
+        const float room = (float)((q.room - fabs(d)) * (1.0 - 0x1p-20));
+        x.end = __shfl((float)(q.end + d), from);
         x.room = fminf(x.room, __shfl(room, from));
-        const int binade = __shfl(r.binade, from);
-        x.binade = x.binade < 0 || at < 0 ? -1 : max(x.binade, binade);
+        x.binade = x.binade < 0 || at < 0 ? -1 : max(x.binade, binade[s][from & 15]);
     }
     if (j == 0) wk.groups[((size_t)c * wk.ngroups + g) * kRcStarts + row] = x;
 }
 
 __global__ __launch_bounds__(256) void k_rc_join(const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                  int nfe, double mass_fe, double mass_si, RcWork wk) {
-    __shared__ RcRun group[kRcMaxGroups][kRcStarts];
-    __shared__ RcRun one[kRcGroup][kRcStarts];  // the runs of a group that does not hold
+    __shared__ RcCand group[kRcMaxGroups][kRcStarts];
+    __shared__ RcCand one[kRcGroup][kRcStarts];  // the runs of a group that does not hold
     __shared__ float guess[kRcMaxRuns];
     __shared__ double terms[64];
     const int c = blockIdx.x;
     const RcRun* __restrict__ runs = wk.runs + (size_t)c * wk.nwin * kRcStarts;
     const int ngroups = wk.ngroups;
     for (int s = threadIdx.x; s < wk.nwin; s += 256) guess[s] = wk.guess[c * wk.nwin + s];
-    for (int k = threadIdx.x; k < ngroups * kRcStarts; k += 256)
-        group[0][k] = wk.groups[(size_t)c * ngroups * kRcStarts + k];
+    __syncthreads();
+    for (int k = threadIdx.x; k < ngroups * kRcStarts; k += 256) {
+        const int g = k / kRcStarts, j = k % kRcStarts;
+        group[g][j] = rc_cand(wk.groups[(size_t)c * ngroups * kRcStarts + k], rc_start(guess[g * kRcGroup], j));
+    }
     __syncthreads();
     if (threadIdx.x >= 64) return;
     const int lane = threadIdx.x, j = lane % kRcStarts;
     const int* __restrict__ bound = wk.bound + c * (wk.nwin + 1);
-    float a = 0.0f;
-    // a joined with run (or group) r from start guess gs: whether it holds
-    auto take = [&](const RcRun& r, float gs) {
+    double a = 0.0;  // a float throughout
+    // a joined with a run (or group): whether it holds, from any of its starts
+    // (the rows of lanes agree)
+    auto take = [&](const RcCand& q) {
         double d;
-        const unsigned m = (unsigned)__ballot(rc_holds(a, rc_start(gs, j), r, d)) & 0xffffu;  // the rows agree
+        const unsigned m = (unsigned)__ballot(rc_holds(a, q, d)) & 0xffffu;
         if (!m) return false;
-        a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int((float)((double)r.end + d)), __builtin_ctz(m)));
+        const double e = (double)(float)(q.end + d);
+        const int at = __builtin_ctz(m);
+        a = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(e), at),
+                             __builtin_amdgcn_readlane(__double2loint(e), at));
         return true;
     };
-    RcRun r = group[0][j];
-    float gs = guess[0];
-    for (int q = 0; q < ngroups; ++q) {
-        const RcRun nr = group[min(q + 1, ngroups - 1)][j];  // the next group's, on its way
-        const float ngs = guess[min(q + 1, ngroups - 1) * kRcGroup];
-        const bool held = take(r, gs);
-        r = nr;
-        gs = ngs;
+    RcCand q = group[0][j];
+    for (int g = 0; g < ngroups; ++g) {
+        const RcCand next = group[min(g + 1, ngroups - 1)][j];  // on its way
+        const bool held = take(q);
+        q = next;
         if (held) continue;
-        const int s0 = q * kRcGroup, s1 = min(s0 + kRcGroup, wk.nwin);
+        const int s0 = g * kRcGroup, s1 = min(s0 + kRcGroup, wk.nwin);
         wave_lds_sync();
-        for (int k = lane; k < (s1 - s0) * kRcStarts; k += 64) one[0][k] = runs[s0 * kRcStarts + k];
+        for (int k = lane; k < (s1 - s0) * kRcStarts; k += 64)
+            one[0][k] = rc_cand(runs[s0 * kRcStarts + k], rc_start(guess[s0 + k / kRcStarts], j));
         const int edge = bound[min(s0 + lane, wk.nwin)];  // lanes 0..kRcGroup
         wave_lds_sync();
         for (int s = s0; s < s1; ++s) {
-            if (take(one[s - s0][j], guess[s])) continue;
+            if (take(one[s - s0][j])) continue;
             const int e = __shfl(edge, s + 1 - s0);
             for (int k0 = __shfl(edge, s - s0); k0 < e; k0 += 64) {
                 wave_lds_sync();
@@ -2194,11 +2236,11 @@ __global__ __launch_bounds__(256) void k_rc_join(const float4* __restrict__ pos,
                 terms[lane] = k0 + lane < e ? (double)rc_value(pos, vel, c, k) * (k < nfe ? mass_fe : mass_si) : -0.0;
                 wave_lds_sync();
 #pragma unroll 8
-                for (int u = 0; u < 64; ++u) a = (float)((double)a + terms[u]);
+                for (int u = 0; u < 64; ++u) a = (double)(float)(a + terms[u]);
             }
         }
     }
-    if (lane == 0) wk.total[c] = a;
+    if (lane == 0) wk.total[c] = (float)a;
 }
 
 __global__ void k_recenter_ref_apply(float4* __restrict__ pos, float4* __restrict__ vel, int n,
