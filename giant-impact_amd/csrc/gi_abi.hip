@@ -1979,7 +1979,7 @@ int gi_find_earth_moon(const gi_float4* pos, const gi_float4* vel, int n, int nf
     hipLaunchKernelGGL(k_scan_add, dim3(nblk(m, 256)), dim3(256), 0, st, w.starts.p, (int)m, w.block_sums.p);
     hipLaunchKernelGGL(k_cc_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, P, n, w.cellhash.p, w.starts.p, w.counts.p,
                        w.spos.p);
-    hipLaunchKernelGGL(k_cc_local, dim3(nblk(n, kCCLocal)), dim3(kCCLocal), 0, st, w.spos.p, n, inv_c, m - 1, touch,
+    hipLaunchKernelGGL(k_cc_local, dim3(nblk(n, kCCLocal)), dim3(kCCLocal * kCCLocalLanes), 0, st, w.spos.p, n, inv_c, m - 1, touch,
                        w.starts.p, w.parent.p);
     hipLaunchKernelGGL(k_cc_union, dim3(nblk(n, kCCUnionPer)), dim3(64 * kCCUnionWaves), 0, st, w.spos.p, n, inv_c,
                        m - 1, touch, w.starts.p, w.parent.p);

@@ -125,11 +125,16 @@ __device__ __forceinline__ int cc_union(int* parent, int a, int b) {
 // so most touching pairs lie in one workgroup's run of kCCLocal particles:
 // k_cc_local unites those in LDS and leaves each particle pointing at the
 // smallest index of its local group; k_cc_union then unites the pairs that
-// cross runs, a lane per (particle, row of cells).  N = 65,536: 46 + 54 us;
-// every pair united globally, five lanes a particle 136-166 us, one lane over
-// all 27 cells with an index load per candidate 350 us.
+// cross runs, a lane per (particle, row of cells).  N = 65,536: 22 + 64 us, and
+// 197 us a call; runs of 512 with a lane per particle 45 + 53 us and 222 a
+// call, of 512 with two 27 + 56, of 256 with two 25 + 65 and 203 a call; every
+// pair united globally, five lanes a particle 136-166 us, one lane over all 27
+// cells with an index load per candidate 350 us.  (In k_cc_union, one union
+// per pair of groups in a wavefront, or four candidates' loads in flight with
+// their groups looked up beside them: 62 and 77 us.)
 constexpr int kCCRows = 5;
-constexpr int kCCLocal = 512;  // particles of a run; lanes of k_cc_local
+constexpr int kCCLocal = 320;     // particles of a run
+constexpr int kCCLocalLanes = 3;  // lanes per particle of k_cc_local, which share its rows
 
 // Buckets of row `row` (0..4) of the cell (cx, cy, cz): candidates
 // [k0[o], k1[o]).  t: the particle's own place.
@@ -159,27 +164,33 @@ __device__ __forceinline__ int cc_lds_find(int* parent, int x) {
     return x;
 }
 
-__global__ __launch_bounds__(kCCLocal) void k_cc_local(const float4* __restrict__ spos, int n, double inv_c,
+__global__ __launch_bounds__(kCCLocal * kCCLocalLanes) void k_cc_local(const float4* __restrict__ spos, int n, double inv_c,
                                                        unsigned hmask, float touch, const int* __restrict__ starts,
                                                        int* __restrict__ parent) {
     __shared__ float4 sp[kCCLocal];
     __shared__ int up[kCCLocal], least[kCCLocal];
     const int b0 = blockIdx.x * kCCLocal, b1 = min(b0 + kCCLocal, n);
-    const int l = threadIdx.x, t = b0 + l;
+    const int l = threadIdx.x % kCCLocal, part = threadIdx.x / kCCLocal, t = b0 + l;
     const bool live = t < n;
     const float4 pi = live ? spos[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const int i = __float_as_int(pi.w);
-    sp[l] = pi;
-    up[l] = l;
-    least[l] = 0x7fffffff;
+    if (part == 0) {
+        sp[l] = pi;
+        up[l] = l;
+        least[l] = 0x7fffffff;
+    }
     __syncthreads();
     if (live) {
         const int cx = cc_cell(pi.x, inv_c), cy = cc_cell(pi.y, inv_c), cz = cc_cell(pi.z, inv_c);
-        int k0[kCCRows][3], k1[kCCRows][3];  // all the bounds' loads in flight at once
+        constexpr int rows = (kCCRows + kCCLocalLanes - 1) / kCCLocalLanes;  // of this lane's rows part, part + lanes, ...
+        int k0[rows][3] = {}, k1[rows][3] = {};  // all the bounds' loads in flight at once
 #pragma unroll
-        for (int row = 0; row < kCCRows; ++row) cc_row(cx, cy, cz, row, t, hmask, starts, k0[row], k1[row]);
+        for (int row = 0; row < rows; ++row) {
+            const int r = part + row * kCCLocalLanes;
+            if (r < kCCRows) cc_row(cx, cy, cz, r, t, hmask, starts, k0[row], k1[row]);
+        }
 #pragma unroll
-        for (int row = 0; row < kCCRows; ++row) {
+        for (int row = 0; row < rows; ++row) {
 #pragma unroll
             for (int o = 0; o < 3; ++o)
                 for (int k = max(k0[row][o], b0); k < min(k1[row][o], b1); ++k) {
@@ -203,10 +214,9 @@ __global__ __launch_bounds__(kCCLocal) void k_cc_local(const float4* __restrict_
         }
     }
     __syncthreads();
-    const int r = cc_lds_find(up, l);
-    if (live) atomicMin(&least[r], i);
+    if (live && part == 0) atomicMin(&least[cc_lds_find(up, l)], i);
     __syncthreads();
-    if (live) parent[i] = least[r];
+    if (live && part == 0) parent[i] = least[cc_lds_find(up, l)];
 }
 
 constexpr int kCCUnionWaves = 4;

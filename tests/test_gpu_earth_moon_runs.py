@@ -1,5 +1,5 @@
 """The Earth / Moon finder at the edges of its workgroups' runs: one to a few
-elements, 512 elements (united in LDS) and 1,024 (sizes counted together) one
+elements, 320 elements (united in LDS) and 1,024 (sizes counted together) one
 less and one more, mostly one group and mostly loners.  Whole numbers equal
 the oracle's, the FP64 sums its FP64 twin's to 1e-9."""
 from __future__ import annotations
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("density", [1.2, 0.08])
-@pytest.mark.parametrize("n", [1, 2, 63, 511, 512, 513, 1023, 1025, 6001])
+@pytest.mark.parametrize("n", [1, 2, 63, 319, 320, 321, 511, 512, 513, 641, 1023, 1025, 6001])
 def test_runs_and_loners(gpu, oracle, n, density):
     rng = np.random.default_rng(n)
     pos, vel = f4(n), f4(n)
