@@ -1326,13 +1326,18 @@ static int launch_recenter(DevCtx* ctx, float4* pos, float4* vel, int n, int nfe
     return 0;
 }
 
-// The reference-float recenter's scratch for n particles, laid out in one
-// buffer of the device's context.  Windows of 64 particles, doubled until
-// one workgroup joins a chain's runs.
+// The reference-float recenter's scratch, laid out in one buffer of the
+// device's context.  Windows of 64 particles, doubled until one workgroup
+// joins a chain's runs.  The buffer (2.1 MB) is made once, for the most runs
+// there can be: a caller may hold a graph of gi_recenter_float, and a later
+// call with more particles must neither move what that graph writes nor
+// allocate under a capture of its own.
 static int recenter_ref_scratch(DevCtx* ctx, int n, RcWork* wk) {
     wk->window = 64;
     while (nblk(n, wk->window) > kRcMaxRuns) wk->window *= 2;
-    const size_t w = wk->nwin = nblk(n, wk->window), groups = wk->ngroups = nblk(wk->nwin, kRcGroup);
+    wk->nwin = nblk(n, wk->window);
+    wk->ngroups = nblk(wk->nwin, kRcGroup);
+    constexpr size_t w = kRcMaxRuns, groups = kRcMaxGroups;
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t o = at;
