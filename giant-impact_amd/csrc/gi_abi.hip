@@ -596,13 +596,6 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
 static std::atomic<int> g_contact_overlap{1};  // see gi_set_contact_overlap
 static std::atomic<int> g_contact_walk{0};     // see gi_set_contact_walk
 
-// The contact walk of plans of up to this many pairs (a simulation of 49,152
-// particles, or several smaller ones) uses nine lanes per particle: their
-// all-pairs pass, up to 0.4 ms, is too short to hide a one-lane walk of 0.2
-// to 0.4 ms and the grid before it (eight simulations of 77,000 particles
-// together, a pass of 0.26 ms: 0.275 ms a step with nine lanes, 0.285 with one).
-constexpr double kContactRowLanesMaxPairs = 49152.0 * 49152.0;
-
 static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched, Plan* out) {
     Plan p;
     p.caller_sims = sims;
@@ -704,10 +697,14 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
     }
     p.overlap_allowed = g_contact_overlap.load() != 0;
     p.contact_walk = g_contact_walk.load();
-    double pairs = 0.0;
+    double particles = 0.0, pairs = 0.0;
     for (const SimDesc& s : sims)
-        if (s.active) pairs += (double)(s.end - s.start) * (double)(s.end - s.start);
-    p.contact_lanes = p.contact_walk ? p.contact_walk : (pairs <= kContactRowLanesMaxPairs ? kCellRows : 1);
+        if (s.active) {
+            const double n = s.end - s.start;
+            particles += n;
+            pairs += n * n;
+        }
+    p.contact_lanes = p.contact_walk ? p.contact_walk : (contact_walk_by_rows(particles, pairs) ? kCellRows : 1);
     p.split_finish = p.mutual && p.tasks.empty() && !p.direct && p.overlap_allowed;
     p.sims = std::move(sims);
     *out = std::move(p);

@@ -151,4 +151,20 @@ inline Tiling choose_tiling(long long ntot, long long pairs, int nsims) {
     return t;
 }
 
+// Whether the contact walk of a plan of so many particles and pairs (sum
+// n^2) takes nine lanes per particle.  One lane's walk is a chain of 27 cells
+// that the all-pairs pass hides only if it is long enough; nine lanes take a
+// ninth of the time and more of the chip, which a pass that fills it pays
+// for.  Measured as whole steps of 8 to 384 equal simulations of 1,100 to
+// 12,000 particles, nine lanes against one: 1.75 times as fast for 8 of 2,048
+// (16,384 particles), 1.23 for 32 of 4,096, 1.07 for 96 of 3,000, 1.03 for 64
+// of 4,096, 1.05 for 16 of 8,000, 1.13 for 8 of 12,000; the same for 192 of
+// 2,048, 128 of 3,000, 96 of 4,096, 32 of 8,000 and 16 of 12,000; 0.90 for
+// 384 of 2,048, 0.96 for 256 of 4,096, 0.97 for 48 of 8,000, 0.98 for 64 of
+// 12,000.  The line through those; one simulation, whose pass is the shorter
+// for its particles, to 49,152.
+inline bool contact_walk_by_rows(double particles, double pairs) {
+    return pairs <= 49152.0 * 49152.0 && particles / 450000.0 + pairs / 3.0e9 <= 1.0;
+}
+
 }  // namespace gi

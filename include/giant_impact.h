@@ -407,8 +407,9 @@ int gi_set_dispatch_limit(long long max_tasks);
 int gi_set_contact_overlap(int enable);
 
 /* Contact walk (lanes = 0, the default: nine lanes per particle for force
- * evaluations of up to 49,152^2 pairs, one lane per particle above): the
- * contact corrections' walk over a particle's 27 neighbour cells, forced to
+ * evaluations of up to 49,152^2 pairs (sum n^2) and, of many simulations
+ * together, particles / 450,000 + pairs / 3e9 <= 1; one lane per particle
+ * above): the contact corrections' walk over a particle's 27 neighbour cells, forced to
  * one lane per particle (1) or one lane per row of three cells (9).  The two
  * forms share their arithmetic: the corrections are bitwise the same either
  * way.  Process-wide; a plan built under another setting is rebuilt on its
