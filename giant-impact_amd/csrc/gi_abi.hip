@@ -285,10 +285,9 @@ constexpr long long kMutualMaxChunk = 4096;
 // work of a piece of L.  A row's i-side slots are its group's pieces in
 // order, then its diagonal pieces, then its in-group tasks: contiguous, as
 // the sums expect.  In the batched engine each simulation's L is the
-// engine's, shortened to N / batched_piece_div(N) (whole 64-blocks, at least
-// one) for simulations too small to fill the GPU with pieces of the full
-// length: a function of the simulation alone, so its sums are the same in
-// any batch.  In a single-simulation plan the last groups (the shortest
+// engine's, shortened (batched_piece_len) for simulations too small to
+// fill the GPU with pieces of the full length: a function of the simulation
+// alone, so its sums are the same in any batch.  In a single-simulation plan the last groups (the shortest
 // j-ranges, whose pieces sort last) take pieces of L / 2 until they hold
 // kTailPieces pieces of L -- one round of the grouped kernel's resident
 // workgroups on MI355X (256 CUs x 6) -- so the launch drains through
@@ -299,15 +298,6 @@ constexpr long long kMutualMaxChunk = 4096;
 // L / 2 (one 30,000-particle simulation stepped 16% faster, eight mixed ones
 // 2%, the 64-simulation ensemble the same within 0.2%; a quarter and a
 // sixteenth gained less).
-//
-// The divisor: a small company's step lasts as long as its longest tasks, a
-// large one's is the longer the more slots there are.  At 32 throughout (and
-// the lists dealt out as below), eight simulations of 4,000 to 18,600
-// particles step in 256 us, two of up to 16,000 in 172, two of 9,500 in 114,
-// four of 12,300 to 18,000 in 260; as below 220, 100, 88 and 231, and the
-// 64-simulation ensemble the same (4.60 ms; 0.5% slower at 64 throughout).
-// One of 30,000 is 2% faster at 32 than at 48.
-static long long batched_piece_div(long long n) { return n <= 16384 ? 80 : n <= 24576 ? 48 : 32; }
 constexpr long long kTailPieces = 1536;
 constexpr long long kBatchedTailDiv = 8;
 
@@ -317,8 +307,7 @@ static int plan_mutual_groups(const std::vector<SimDesc>& sims, const Tiling& tl
     for (size_t si = 0; si < sims.size(); ++si) {
         const SimDesc& s = sims[si];
         if (s.gn == 0) continue;
-        const long long n = s.end - s.start;
-        const long long L = batched ? std::min(L0, std::max(64LL, (n / batched_piece_div(n) + 63) / 64 * 64)) : L0;
+        const long long L = batched ? batched_piece_len(s.end - s.start, L0) : L0;
         const int nrows = s.gn / B;
         const int fe_real = (s.fe_end - s.start + 63) / 64 * 64;
         const int si_real = s.gfe + (s.end - s.fe_end + 63) / 64 * 64;

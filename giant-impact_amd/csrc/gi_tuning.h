@@ -25,6 +25,7 @@
 
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -134,6 +135,32 @@ inline BatchedTiling batched_tiling() {
     });
     if (from_file.chunk_len > 0) return from_file;
     return BatchedTiling{4096, 1, 0};
+}
+
+// j per piece of a simulation of n particles in the batched engine, whose
+// full length is L0.  A piece costs a slot per particle of its rows, written
+// and added, and a task's start; a company of a few small simulations lasts as
+// long as its longest tasks, a full GPU the longer the more pieces there are.
+// What is in company must not change a simulation's sums, so one length has to
+// do for both.  Steps of equal simulations, against pieces of n / 32 in lists
+// longest first and the walk by particles alone (alone: of a small company,
+// then of a GPU full of them):
+//   64 to 3,072: 2 of 2,600 94 -> 59 us, 150 of them 356 ->
+//     322; up to 4,096 they cost 256 simulations 9%;
+//   n / 40 to 16,384: 2 of 4,501 112 -> 73, 150 759 -> 691; 2 of 9,001 162 ->
+//     95, 150 2,321 -> 2,330; n / 80 takes 85 and 2,469, and 256 simulations
+//     of 4,096 9% longer, 150 of 3,700 to 9,800 3 to 6%;
+//   256 at most there: 2 of 12,701 164 -> 115, 64 1,845 -> 1,876; n / 80 takes
+//     110 and 1,906, n / 48 (320) 3 of 12,700 to 13,600 10% longer than n / 32;
+//     64 simulations of 10,600 to 15,700 1% longer on average, 32 3% shorter;
+//   n / 48 to 24,576: 2 of 23,399 304 -> 257, 16 1,673 -> 1,519, 64 the same
+//     within 0.6%; 3 of 17,600 and 22,500 11 and 4% longer, where the tasks
+//     divide badly among the CUs;
+//   n / 32 above: one of 30,000 is 2% faster so than at n / 48.
+inline long long batched_piece_len(long long n, long long L0) {
+    long long L = n <= 3072 ? 64 : n <= 16384 ? n / 40 : n <= 24576 ? n / 48 : n / 32;
+    if (n <= 16384 && L > 256) L = 256;
+    return std::min(L0, std::max(64LL, (L + 63) / 64 * 64));
 }
 
 // The row for a launch of ntot particles.  Several simulations in one launch

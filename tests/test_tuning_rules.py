@@ -37,3 +37,15 @@ def rule(tmp_path_factory):
 ])
 def test_contact_walk(rule, sims, n, lanes):
     assert rule("walk", sims, n) == lanes
+
+
+# (particles, the engine's length, j per piece): the longest length, or within
+# 1-2% of the fastest, for a full GPU of such simulations
+@pytest.mark.parametrize("n,full,length", [
+    (1, 768, 64), (2048, 768, 64), (3072, 768, 64), (3073, 768, 128), (4096, 768, 128), (5120, 768, 128),
+    (6000, 768, 192), (7000, 768, 192), (8000, 768, 256), (10000, 768, 256), (12000, 768, 256), (16384, 768, 256),
+    (16385, 768, 384), (20000, 768, 448), (24576, 768, 512), (24577, 768, 768), (65536, 768, 768),
+    (65536, 4096, 2048), (8000, 128, 128), (20000, 64, 64),
+])
+def test_batched_piece(rule, n, full, length):
+    assert rule("piece", n, full) == length
