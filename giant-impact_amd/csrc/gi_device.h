@@ -179,7 +179,8 @@ __device__ __forceinline__ float approach_k(const PairLaw& L, int test) {
 // rounding error of every addition, whichever operand is the larger, is
 // carried in c, so a long sum of floats keeps float precision of its result
 // instead of losing it with the number of terms.  The force path accumulates
-// in it; FP64 is kept for the energy and angular-momentum reductions.
+// in it; FP64 is kept for the energy and angular-momentum reductions and, where
+// there are few of them, the direct pass's sums.
 struct CompSum {
     float s, c;
     __device__ __forceinline__ void zero() { s = c = 0.0f; }
@@ -192,12 +193,6 @@ struct CompSum {
     __device__ __forceinline__ void add_sum(const CompSum& o) {
         add(o.s);
         c += o.c;
-    }
-    // the product a * b, its rounding error (exact, by FMA) carried over
-    __device__ __forceinline__ void add_product(float a, float b) {
-        const float p = a * b;
-        add(p);
-        c += __builtin_fmaf(a, b, -p);
     }
     __device__ __forceinline__ float value() const { return s + c; }
 };

@@ -1146,31 +1146,38 @@ __global__ __launch_bounds__(64 * kContactWaves) void k_contact_corr(int ntot, c
 // is kDirectI independent chains.  (With the lanes over i and the j's
 // broadcast to them, each 64 pairs took a 16-byte load per lane: 16 cycles of
 // a CU's load path, which bounded the kernel: a step of N = 2,048, 4,096,
-// 8,192 and 11,000 took 11.9, 20.4, 50.6 and 117 us, and takes 8.0, 12.6,
-// 29.1 and 51.)  It is bound by vector issue, 16 instructions per 64 pairs,
+// 8,192 and 11,000 took 12.0, 20.1, 49.7 and 116 us, and takes 7.8, 12.7,
+// 29.7 and 50.8.)  It is bound by vector issue, 16 instructions per 64 pairs,
 // at the large end (11,000: 70% of the issue rate) and by the chain of loads,
 // step, contact terms and sums at the small end.  A wavefront's j are of one
 // material (the wavefronts are divided between the iron and the silicate j),
 // so the gravity product is one factor per wavefront and i.  Every pair takes
 // the all-pairs pass's branch-free gravity term into a float sum per lane and
-// i (N / 64 W terms for W wavefronts), added over the lanes as a tree.
+// i, of at most kDirectFold terms; four lanes' sums are added in float, all
+// beyond in FP64.
 //
 // Pairs with r^2 < 1 are listed as they are met, in j order, one list per
 // wavefront; a full list and at the end what is left is worked off a pair per
 // lane: the exact contact term minus the gravity term, with the arithmetic of
-// k_finish, added per i in list order in a compensated sum.  The wavefronts'
-// sums are added in a compensated float sum in a fixed order, so the result
-// depends on the simulation alone.
+// k_finish, added in FP64.  The wavefronts' sums are added in FP64 in a fixed
+// order and rounded once, so the result depends on the simulation alone.
+// (64 lanes folded in float and the contact terms of a batch too, with
+// compensated sums between: the whole error, which v_rsq sets, was 1.0 to
+// 1.9% larger in contact states and up to 0.15% in others, N = 300 to 12,288,
+// than with every sum compensated; as it is, within 0.1% of that.  FP64 costs
+// 0.2 us a call up to N = 2,048 and 2.5 to 4% above.)
 //
 // Eight wavefronts per workgroup, so that another has room beside the running
-// ones: a call takes 5.4, 6.6, 9.6 and 18.0 us at N = 1,024, 2,048, 3,072 and
-// 6,000, with 16 wavefronts 5.8, 6.7, 11.7 and 23.5 (four were slower up to
-// 8,192 and even above).
+// ones: a call takes 5.7, 7.0, 10.4 and 19.3 us at N = 1,024, 2,048, 3,072 and
+// 6,000 (before the FP64 sums 5.5, 6.8, 9.9 and 18.5, and with 16 wavefronts
+// 5.8, 6.7, 11.7 and 23.5; four were slower up to 8,192 and even above).
 constexpr int kDirectI = 8;
 constexpr int kDirectForceWaves = 8;
 // r^2 (with FMAs and kSelfEps) of every pair whose exactly rounded r is below
 // 1 lies below this: the margin covers the few ulps between the two forms.
 constexpr float kDirectContactR2 = 1.0001f;
+// 64-blocks a wavefront's float sums run over.
+constexpr int kDirectFold = 64;
 
 // The move of a step fused into the direct pass (MOVE = 1:
 // moveBodiesCollisionSingleGPU, impactAddTime.cu:379-394; MOVE = 2:
@@ -1190,6 +1197,25 @@ template <int CTRL>
 __device__ __forceinline__ float lane_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
+template <int CTRL>
+__device__ __forceinline__ double lane_dpp(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
+}
+// The lower 32 lanes get x of themselves plus x of lane + 32, the upper 32 y of
+// lane - 32 plus y of themselves; for SPAN = 16, of each pair of rows of lanes.
+template <int SPAN>
+__device__ __forceinline__ double halves_sum(double x, double y) {
+    if constexpr (SPAN == 32) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(y), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(y), false, false);
+        return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    } else {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(y), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(y), false, false);
+        return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+}
 // lanes with `hi` keep y and send x to their partner, the others keep x
 template <int CTRL>
 __device__ __forceinline__ float lane_fold(float x, float y, bool hi) {
@@ -1197,33 +1223,27 @@ __device__ __forceinline__ float lane_fold(float x, float y, bool hi) {
     return keep + lane_dpp<CTRL>(send);
 }
 // x[k] summed over the 16 lanes of each row of lanes; lane p of the row gets
-// the sum of x[p & 7].
-__device__ __forceinline__ float row_sums8(const float (&x)[8], int p) {
+// the sum of x[p & 7].  Four lanes' sums are added in float, then FP64.
+__device__ __forceinline__ double row_sums8(const float (&x)[8], int p) {
     float a[4], b[2];
 #pragma unroll
     for (int k = 0; k < 4; ++k) a[k] = lane_fold<0x141>(x[k], x[k + 4], p & 4);  // lane p with 7 - p of its half row
 #pragma unroll
     for (int k = 0; k < 2; ++k) b[k] = lane_fold<0x4E>(a[k], a[k + 2], p & 2);  // with p ^ 2
-    const float c = lane_fold<0xB1>(b[0], b[1], p & 1);                         // with p ^ 1
-    return c + lane_dpp<0x128>(c);                                              // with p ^ 8
+    const bool hi = p & 1;
+    const double c = (double)(hi ? b[1] : b[0]) + (double)lane_dpp<0xB1>(hi ? b[0] : b[1]);  // with p ^ 1
+    return c + lane_dpp<0x128>(c);                                                           // with p ^ 8
 }
 // The four rows' x, y and z added: row 0 gets x, row 1 y, row 2 z.
-__device__ __forceinline__ float rows_sum_xyz(float x, float y, float z) {
-    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(z), false, false);
-    const float xz = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), 0u, false, false);
-    const float y0 = __uint_as_float(t[0]) + __uint_as_float(t[1]);
-    const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(xz), __float_as_uint(y0), false, false);
-    return __uint_as_float(u[0]) + __uint_as_float(u[1]);
+__device__ __forceinline__ double rows_sum_xyz(double x, double y, double z) {
+    return halves_sum<16>(halves_sum<32>(x, z), halves_sum<32>(y, 0.0));
 }
 
 // x summed over the lanes 8 p + k of each k, on every lane.
-__device__ __forceinline__ float eighths_sum(float x) {
+__device__ __forceinline__ double eighths_sum(double x) {
     x += lane_dpp<0x128>(x);
-    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+    x = halves_sum<16>(x, x);
+    return halves_sum<32>(x, x);
 }
 
 // Four float4 records in one load.
@@ -1240,8 +1260,8 @@ __global__ __launch_bounds__(64 * kDirectForceWaves) void k_direct(const float4*
     constexpr int IB = kDirectI;
     constexpr int kWorkOff = 128;             // listed pairs that are worked off before the next step
     constexpr int kList = kWorkOff + 64 * IB;  // and what one step can add
-    __shared__ float grav[W][4 * 16];     // per wavefront: row c, lane p -> component c of i p
-    __shared__ float contact[W][6][IB];   // per wavefront: (sum, compensation) of x, y, z
+    __shared__ double grav[W][4 * 16];    // per wavefront: row c, lane p -> component c of i p
+    __shared__ double contact[W][3][IB];
     __shared__ int list[W][kList];        // i << 24 | j
     __shared__ float4 term[W][64];
     const int lane = threadIdx.x & 63;
@@ -1284,13 +1304,12 @@ __global__ __launch_bounds__(64 * kDirectForceWaves) void k_direct(const float4*
     float ax[IB], ay[IB], az[IB];
 #pragma unroll
     for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
-    CompSum cx, cy, cz;  // lane 8 p + k: the contact terms of i k
-    cx.zero();
-    cy.zero();
-    cz.zero();
+    double gsum = 0.0;                     // the folded tiles: row c, lane p -> component c of i p
+    double cx = 0.0, cy = 0.0, cz = 0.0;  // lane 8 p + k: contact terms of i k
     int listed = 0;
+    int jt = min(je, jb + kDirectFold * stride);  // the tile's end
     for (;;) {
-        while (jb < je && listed <= kWorkOff) {
+        while (jb < jt && listed <= kWorkOff) {
             float4 pj = nx;
             const int j0 = jb;
             jb += stride;
@@ -1360,38 +1379,35 @@ __global__ __launch_bounds__(64 * kDirectForceWaves) void k_direct(const float4*
             }
             term[wv][lane] = t;
             wave_lds_sync();
-            // A batch's terms of one i, a handful, in plain float sums: lane
-            // 8 p + k takes those of i k among every eighth term, then the
-            // eight lanes of an i are added.  (All 64 terms looked at by each
-            // of eight lanes took 1 us a batch: a step of N = 1,024 in
-            // contact 9.3 us, 7.0 so, of 8,192 33.5 and 29.6.)
-            float bx = 0.0f, by = 0.0f, bz = 0.0f;
+            // Lane 8 p + k takes the terms of i k among every eighth term of
+            // the batch.  (All 64 terms looked at by each of eight lanes took
+            // 1 us a batch: a step of N = 1,024 in contact 9.3 us, 7.0 so, of
+            // 8,192 33.5 and 29.6.)
 #pragma unroll 4
             for (int u = 0; u < 8; ++u) {
                 const float4 o = term[wv][8 * u + (lane >> 3)];
                 const bool mine = __float_as_int(o.w) == (lane & 7);
-                bx += mine ? o.x : 0.0f;
-                by += mine ? o.y : 0.0f;
-                bz += mine ? o.z : 0.0f;
+                cx += (double)(mine ? o.x : 0.0f);
+                cy += (double)(mine ? o.y : 0.0f);
+                cz += (double)(mine ? o.z : 0.0f);
             }
-            bx = eighths_sum(bx);
-            by = eighths_sum(by);
-            bz = eighths_sum(bz);
-            cx.add(bx);
-            cy.add(by);
-            cz.add(bz);
         }
-        if (jb >= je) break;
         listed = 0;
+        if (jb < jt) continue;
+        gsum += rows_sum_xyz(row_sums8(ax, lane & 15), row_sums8(ay, lane & 15), row_sums8(az, lane & 15));
+        if (jb >= je) break;
+        jt = min(je, jb + kDirectFold * stride);
+#pragma unroll
+        for (int k = 0; k < IB; ++k) ax[k] = ay[k] = az[k] = 0.0f;
     }
-    grav[wv][lane] = rows_sum_xyz(row_sums8(ax, lane & 15), row_sums8(ay, lane & 15), row_sums8(az, lane & 15));
+    grav[wv][lane] = gsum;
+    cx = eighths_sum(cx);
+    cy = eighths_sum(cy);
+    cz = eighths_sum(cz);
     if (lane < IB) {
-        contact[wv][0][lane] = cx.s;
-        contact[wv][1][lane] = cx.c;
-        contact[wv][2][lane] = cy.s;
-        contact[wv][3][lane] = cy.c;
-        contact[wv][4][lane] = cz.s;
-        contact[wv][5][lane] = cz.c;
+        contact[wv][0][lane] = cx;
+        contact[wv][1][lane] = cy;
+        contact[wv][2][lane] = cz;
     }
     // Wavefront c < 3 adds component c: lane w * 8 + k takes the sums of i k
     // of wavefront w, then the eight lanes of an i are added.  The move's
@@ -1416,20 +1432,9 @@ __global__ __launch_bounds__(64 * kDirectForceWaves) void k_direct(const float4*
             }
         return;
     }
-    CompSum t;
-    t.zero();
-    t.add_product(g, grav[w][16 * wv + k]);
-    t.add(contact[w][2 * wv][k]);
-    t.c += contact[w][2 * wv + 1][k];
-#pragma unroll
-    for (int m = 8; m < 64; m <<= 1) {
-        CompSum o;
-        o.s = __shfl_xor(t.s, m);
-        o.c = __shfl_xor(t.c, m);
-        t.add_sum(o);
-    }
+    const double sum = eighths_sum((double)g * grav[w][16 * wv + k] + contact[w][wv][k]);
     if (lane >= IB || i >= end) return;
-    const float f = t.value();
+    const float f = (float)sum;
     reinterpret_cast<float*>(force + i)[wv] = f;
     if constexpr (MOVE != 0) {
         float temp, damp = 0.0f;
