@@ -121,8 +121,8 @@ struct Plan {
     bool overlap_allowed = true;  // gi_set_contact_overlap when planned
     int contact_lanes = 1;        // lanes per particle of the contact walk (1 or 9)
     int contact_walk = 0;         // gi_set_contact_walk when planned
-    // direct pass (tiling.variant == 3): one workgroup per 64 / direct_lanes
-    // i-particles
+    // direct pass (tiling.variant == 3): a block table entry per
+    // 64 / direct_lanes i-particles
     bool direct = false;
     int direct_lanes = 1;
     std::vector<DirectBlock> dblocks;
@@ -608,7 +608,8 @@ static int build_plan(std::vector<SimDesc> sims, const Tiling& tl, bool batched,
         if (rc < 0) return rc;
     }
     if (tl.variant == 3) {
-        // R = lanes per i-particle (j-streams per wavefront): 1, 2, 4 or 8
+        // R = lanes per i-particle of the energy pass; the force takes eight
+        // i-particles of an entry per workgroup whatever R is
         p.direct_lanes = std::min(tl.R, 8);
         const int ib = 64 / p.direct_lanes;
         for (size_t si = 0; si < sims.size(); ++si)
@@ -1528,7 +1529,7 @@ namespace gi {
 // ---------------------------------------------------------------------------
 
 constexpr int kNoAllocMaxN = 12288;                    // particles per call, at most
-constexpr int kNoAllocMaxBlocks = kNoAllocMaxN / 8;  // >= 8 i-particles per workgroup
+constexpr int kNoAllocMaxBlocks = kNoAllocMaxN / 8;  // >= 8 i-particles per entry
 struct NoAllocScratch {
     SimDesc sim;
     DirectBlock blocks[kNoAllocMaxBlocks];
@@ -1543,7 +1544,7 @@ static std::mutex g_noalloc_mutex;
 static NoAllocScratch* g_noalloc_ptr[64];  // per device, set once
 
 // Writes the descriptor and the block table of one simulation of n
-// particles, ib i-particles per workgroup.
+// particles, ib i-particles per entry.
 __global__ void k_noalloc_plan(NoAllocScratch* __restrict__ s, SimDesc sd, int nb, int ib, int iron_waves) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) s->sim = sd;
@@ -1812,8 +1813,8 @@ int gi_force_collision_noalloc(const gi_float4* pos, const gi_float4* vel, gi_fl
         }
         sp = g_noalloc_ptr[dev];
     }
-    // The direct pass with the tuning table's lanes per particle for this n
-    // (the plan gi_force_collision makes where the table picks that pass).
+    // The direct pass with the tuning table's block table for this n (the plan
+    // gi_force_collision makes where the table picks that pass).
     const Tiling t = choose_tiling(n, (long long)n * n, 1);
     const int lanes = t.variant == 3 ? std::min(t.R, 8) : 1;
     const int ib = 64 / lanes;

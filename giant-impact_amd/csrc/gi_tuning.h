@@ -5,8 +5,8 @@
 //              rcp (1 multiply, 2 transcendental ops); 2 = mutual pass (each
 //              pair once for both particles, rows of 64*R, rsq cubed);
 //              3 = direct pass (small simulations: the whole force in one
-//              launch; 64 / R i-particles per workgroup, R = 1, 2, 4 or 8;
-//              the sizes unused);
+//              launch, the same whatever R is; R = 1, 2, 4 or 8 lanes per
+//              particle of its energy pass; the sizes unused);
 //              4 = mutual pass with row groups (a workgroup's four
 //              wavefronts hold four rows and add their j-side sums in LDS
 //              before writing them: a quarter of the j-side slab; R = 4 or 8)
@@ -19,7 +19,7 @@
 // The table is written by the autotuner (gi_amd.autotune) to
 // tuning/<arch>.txt next to the library's lib/ directory, one row per size
 // class: "n_max R variant chunk_len target_tasks min_chunk" (particles of
-// the whole launch, rows in increasing n_max).  Without a table the defaults
+// one simulation, or sqrt(sum n^2) of several; rows in increasing n_max).  Without a table the defaults
 // below apply.
 #pragma once
 

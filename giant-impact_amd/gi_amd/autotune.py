@@ -6,9 +6,12 @@ correction, or the direct pass alone) over a grid of tilings -- the
 one-sided pass with R (i-particles per lane), the r^-3 variant and the
 number of wavefront tasks, the mutual pass (variant 2) and its row-group form
 (variant 4) with R (rows of 64*R) and their chunk length, and for the small
-classes the direct pass (variant 3)
--- and writes the fastest to tuning/gfx950.txt, which libgiant_impact.so
-reads on first use:
+classes the direct pass (variant 3) -- and writes the fastest to
+tuning/gfx950.txt, which libgiant_impact.so reads on first use.  The direct
+pass's force is the same whatever its R, which is the energy pass's lanes per
+particle: where the direct pass wins, R is the fastest for
+gi_conserved_quantities.
+
 
     n_max R variant chunk_len target_tasks min_chunk
 
@@ -25,7 +28,7 @@ from pathlib import Path
 
 import numpy as np
 
-from . import DeviceArray, call, device_count, force_collision, load, make_impact, sync
+from . import DeviceArray, call, conserved_quantities, device_count, force_collision, load, make_impact, sync
 
 TUNING_DIR = Path(__file__).resolve().parent.parent / "tuning"
 
@@ -49,6 +52,17 @@ CLASSES = [
 DIRECT_MAX_CLASS = 49152
 
 
+def candidates(n_max: int, n: int, Rs, variants, targets, mutual_Ls) -> list:
+    """The tilings timed for a class: (R, variant, chunk_len, target_tasks,
+    min_chunk).  One of the direct pass, whose R does not change the force."""
+    mc = 128 if n < 4096 else 512
+    cands = [(R, v, 0, tt, mc) for R, v, tt in itertools.product(Rs, variants, targets)]
+    cands += [(R, v, L, 0, 64) for R, L, v in itertools.product([4, 8], mutual_Ls, [2, 4])]
+    if n_max <= DIRECT_MAX_CLASS:
+        cands.append((4, 3, 0, 0, 0))
+    return cands
+
+
 def time_gravity(n_target: int, n_impactor: int, reps: int):
     pos, vel, fc, _, _ = make_impact(n_target, n_impactor, seed=77)
     n = len(pos)
@@ -68,7 +82,17 @@ def time_gravity(n_target: int, n_impactor: int, reps: int):
         call("gi_kernel_timing", b"force", C.byref(L), C.byref(T))
         return T.value / max(L.value, 1)
 
-    return run, n
+    def energy() -> float:
+        conserved_quantities(P, V, n, fc)  # plan + warm
+        best = float("inf")
+        for _ in range(5):
+            t0 = time.perf_counter()
+            for _ in range(reps):
+                conserved_quantities(P, V, n, fc)
+            best = min(best, (time.perf_counter() - t0) / reps)
+        return best * 1e3
+
+    return run, energy, n
 
 
 def tune_batched(quick: bool):
@@ -141,13 +165,8 @@ def main(argv=None) -> int:
             if n_max in kept:
                 rows.append(kept[n_max])
             continue
-        run, n = time_gravity(nt, ni, reps=3 if nt + ni > 100000 else 10)
-        mc = 128 if n < 4096 else 512
-        # (R, variant, chunk_len, target_tasks, min_chunk)
-        cands = [(R, v, 0, tt, mc) for R, v, tt in itertools.product(Rs, variants, targets)]
-        cands += [(R, v, L, 0, 64) for R, L, v in itertools.product([4, 8], mutual_Ls, [2, 4])]
-        if n_max <= DIRECT_MAX_CLASS:
-            cands += [(S, 3, 0, 0, 0) for S in (1, 2, 4, 8)]  # R = lanes per i-particle
+        run, energy, n = time_gravity(nt, ni, reps=3 if nt + ni > 100000 else 10)
+        cands = candidates(n_max, n, Rs, variants, targets, mutual_Ls)
         best = None
         for cand in cands:
             call("gi_set_tiling", *cand)
@@ -158,6 +177,13 @@ def main(argv=None) -> int:
             if best is None or ms < best[0]:
                 best = (ms, cand)
         ms, cand = best
+        if cand[1] == 3:
+            lanes = {}
+            for R in Rs:
+                call("gi_set_tiling", R, *cand[1:])
+                lanes[R] = energy()
+                print(f"n={n:8d} R={R} v=3: energy {lanes[R]:9.4f} ms", flush=True)
+            cand = (min(lanes, key=lanes.get),) + cand[1:]
         print(f"# class n<={n_max}: best {cand} ({n * n / (ms / 1e3):.3e} pair/s)", flush=True)
         rows.append((n_max,) + cand)
     call("gi_set_tiling", 0, 0, 0, 0, 0)

@@ -161,7 +161,7 @@ int gi_mem_info(size_t *free_bytes, size_t *total_bytes);
  * when it uses the mutual all-pairs pass (k_mutual) for some simulation, 3
  * for its row-group form (k_mutual_grp), 2 when it uses the direct pass
  * (k_direct), 0 for the one-sided pass (k_gravity); r = i-particles per lane, pair_tasks = wavefront tasks of the
- * all-pairs kernel(s) (workgroups of the direct pass), chunk_len = j per task
+ * all-pairs kernel(s) (block table entries of the direct pass), chunk_len = j per task
  * of the mutual pass.  Zeros before the first call.  Any pointer may be NULL. */
 int gi_plan_info(int *mutual, int *r, long long *pair_tasks, long long *chunk_len);
 
@@ -353,8 +353,8 @@ int gi_find_earth_moon(const gi_float4 *pos, const gi_float4 *vel, int n, int nf
  * lane (1, 2, 4 or 8), variant = the all-pairs pass (0: one-sided, r^-3 as rsq
  * cubed; 1: one-sided, rsq*rcp; 2: mutual -- each pair evaluated once for both
  * particles, rows of 64*r particles; 3: direct -- small simulations, the whole
- * force, contacts included, in one launch, r = 1, 2, 4 or 8: 64 / r
- * i-particles per entry of the block table),
+ * force, contacts included, in one launch, the same whatever r is; r = 1, 2,
+ * 4 or 8 lanes per particle of gi_conserved_quantities' energy pass),
  * chunk_len = j-particles per task (0 =
  * derived from target_tasks),
  * target_tasks = wavefront tasks to aim for, min_chunk = lower bound of
