@@ -1355,11 +1355,15 @@ static int launch_recenter_ref(DevCtx* ctx, float4* pos, float4* vel, int n, int
     int rc;
     if ((rc = recenter_ref_scratch(ctx, n, &wk))) return rc;
     const float4 *P = pos, *V = vel;
-    const dim3 wgrid(nblk(wk.nwin, kRcWindowWaves)), wblock(64 * kRcWindowWaves);
-    hipLaunchKernelGGL(k_rc_window_sums, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
-    hipLaunchKernelGGL(k_rc_bounds, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
-    hipLaunchKernelGGL(k_rc_runs, dim3(kRcChains * wk.ngroups), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
-    hipLaunchKernelGGL(k_rc_join, dim3(kRcChains), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
+    if (n <= kRcStepsMaxN) {
+        hipLaunchKernelGGL(k_rc_steps, dim3(kRcChains), dim3(64), 0, st, P, V, n, nfe, mfe, msi, wk.total);
+    } else {
+        const dim3 wgrid(nblk(wk.nwin, kRcWindowWaves)), wblock(64 * kRcWindowWaves);
+        hipLaunchKernelGGL(k_rc_window_sums, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
+        hipLaunchKernelGGL(k_rc_bounds, wgrid, wblock, 0, st, P, V, n, nfe, mfe, msi, wk);
+        hipLaunchKernelGGL(k_rc_runs, dim3(kRcChains * wk.ngroups), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
+        hipLaunchKernelGGL(k_rc_join, dim3(kRcChains), dim3(256), 0, st, P, V, nfe, mfe, msi, wk);
+    }
     hipLaunchKernelGGL(k_recenter_ref_apply, dim3(nblk(n, 256)), dim3(256), 0, st, pos, vel, n,
                        (const float*)wk.total, tc[0], tc[1], tc[2], tv[0], tv[1], tv[2]);
     GI_HIP(hipGetLastError());

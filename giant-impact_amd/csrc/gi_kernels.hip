@@ -2187,6 +2187,37 @@ __global__ __launch_bounds__(256) void k_rc_runs(const float4* __restrict__ pos,
     if (j == 0) wk.groups[((size_t)c * wk.ngroups + g) * kRcStarts + row] = x;
 }
 
+// Chain c from a on over the elements [k0, e), step by step, by one wavefront:
+// 64 terms at a time through its 64 doubles of LDS.
+__device__ __forceinline__ double rc_chain(const float4* __restrict__ pos, const float4* __restrict__ vel, int c,
+                                           int k0, int e, int nfe, double mass_fe, double mass_si, double a,
+                                           double* __restrict__ terms) {
+    const int lane = threadIdx.x & 63;
+    for (; k0 < e; k0 += 64) {
+        wave_lds_sync();
+        const int k = min(k0 + lane, e - 1);
+        // past the end: -0 leaves every sum as it is
+        terms[lane] = k0 + lane < e ? (double)rc_value(pos, vel, c, k) * (k < nfe ? mass_fe : mass_si) : -0.0;
+        wave_lds_sync();
+#pragma unroll 8
+        for (int u = 0; u < 64; ++u) a = (double)(float)(a + terms[u]);
+    }
+    return a;
+}
+
+// All of a chain step by step, for so few particles that the four launches of
+// the runs cost more than they save.  N = 40, 256, 512, 1,024, 1,536 and
+// 2,048: 8, 8, 12, 19, 27 and 35 us a call and by runs 24, 31, 35, 39, 39 and
+// 45 (bodies in motion: 2,048 40 and 40, 3,000 54 and 43); all seven chains on
+// one wavefront 9, 17, 31, 57, 84 and 110.
+constexpr int kRcStepsMaxN = 2048;
+__global__ __launch_bounds__(64) void k_rc_steps(const float4* __restrict__ pos, const float4* __restrict__ vel, int n,
+                                                 int nfe, double mass_fe, double mass_si, float* __restrict__ total) {
+    __shared__ double terms[64];
+    const double a = rc_chain(pos, vel, blockIdx.x, 0, n, nfe, mass_fe, mass_si, 0.0, terms);
+    if (threadIdx.x == 0) total[blockIdx.x] = (float)a;
+}
+
 __global__ __launch_bounds__(256) void k_rc_join(const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                  int nfe, double mass_fe, double mass_si, RcWork wk) {
     __shared__ RcCand group[kRcMaxGroups][kRcStarts];
@@ -2233,16 +2264,7 @@ __global__ __launch_bounds__(256) void k_rc_join(const float4* __restrict__ pos,
         wave_lds_sync();
         for (int s = s0; s < s1; ++s) {
             if (take(one[s - s0][j])) continue;
-            const int e = __shfl(edge, s + 1 - s0);
-            for (int k0 = __shfl(edge, s - s0); k0 < e; k0 += 64) {
-                wave_lds_sync();
-                const int k = min(k0 + lane, e - 1);
-                // past the run's end: -0 leaves every sum as it is
-                terms[lane] = k0 + lane < e ? (double)rc_value(pos, vel, c, k) * (k < nfe ? mass_fe : mass_si) : -0.0;
-                wave_lds_sync();
-#pragma unroll 8
-                for (int u = 0; u < 64; ++u) a = (double)(float)(a + terms[u]);
-            }
+            a = rc_chain(pos, vel, c, __shfl(edge, s - s0), __shfl(edge, s + 1 - s0), nfe, mass_fe, mass_si, a, terms);
         }
     }
     if (lane == 0) wk.total[c] = (float)a;
