@@ -49,3 +49,14 @@ def test_contact_walk(rule, sims, n, lanes):
 ])
 def test_batched_piece(rule, n, full, length):
     assert rule("piece", n, full) == length
+
+
+# where the class above or below would take single calls longer than the forms
+# that had these sizes before them
+@pytest.mark.parametrize("n,R,variant,length", [
+    (12289, 4, 2, 128), (24576, 4, 2, 128), (24577, 4, 2, 256), (25300, 4, 2, 256), (27600, 4, 2, 256),
+    (33793, 4, 2, 256), (36000, 4, 2, 256), (36353, 8, 4, 128), (49152, 8, 4, 128), (49153, 8, 4, 256),
+])
+def test_mid_size_rows(gi, n, R, variant, length):
+    t = gi.tiling_for(n)
+    assert (t["r"], t["variant"], t["chunk_len"]) == (R, variant, length)
