@@ -38,7 +38,7 @@ CLASSES = [
     (6144, 3072, 1024),
     (12288, 6144, 2048),
     (24576, 13312, 4435),
-    (36352, 24576, 6144),
+    (33792, 24576, 6144),
     (49152, 31488, 10496),
     (98304, 49152, 16384),
     (196608, 98304, 32768),

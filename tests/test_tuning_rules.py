@@ -55,7 +55,7 @@ def test_batched_piece(rule, n, full, length):
 # that had these sizes before them
 @pytest.mark.parametrize("n,R,variant,length", [
     (12289, 4, 2, 128), (24576, 4, 2, 128), (24577, 4, 2, 256), (25300, 4, 2, 256), (27600, 4, 2, 256),
-    (33793, 4, 2, 256), (36000, 4, 2, 256), (36353, 8, 4, 128), (49152, 8, 4, 128), (49153, 8, 4, 256),
+    (33792, 4, 2, 256), (33793, 8, 4, 128), (49152, 8, 4, 128), (49153, 8, 4, 256),
 ])
 def test_mid_size_rows(gi, n, R, variant, length):
     t = gi.tiling_for(n)
