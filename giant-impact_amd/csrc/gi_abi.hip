@@ -524,23 +524,28 @@ static int plan_mutual(std::vector<SimDesc>& sims, const Tiling& tl, bool batche
     // k_mutual_sum's workgroups: the 64-blocks of every row that hold a real
     // particle, heaviest first (a particle adds its row's slots and one slab
     // entry per earlier row).
-    std::vector<SumBlock> sblocks;
-    std::vector<int> swork;
+    struct SumPlace {
+        int work, sim, q0;
+    };
+    std::vector<SumPlace> places;
+    places.reserve((size_t)gb / 64);
     for (size_t si = 0; si < sims.size(); ++si) {
         const SimDesc& s = sims[si];
         if (s.gn == 0) continue;
         const int nfe = s.fe_end - s.start, nsi = s.end - s.fe_end;
         for (int q0 = 0; q0 < s.gn; q0 += 64) {
             if (q0 < s.gfe ? q0 >= nfe : q0 - s.gfe >= nsi) continue;  // ghosts only
-            sblocks.push_back(sum_block(s, (int)si, q0, B, W, rows[s.row0 + q0 / B]));
-            swork.push_back(sblocks.back().nslot + sblocks.back().group + sblocks.back().in_group);
+            const int row = q0 / B;
+            places.push_back(SumPlace{rows[s.row0 + row].nslot + row / W + row % W, (int)si, q0});
         }
     }
-    std::vector<int> order(sblocks.size());
-    for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return swork[a] > swork[b]; });
-    p.sblocks.resize(order.size());
-    for (size_t k = 0; k < order.size(); ++k) p.sblocks[k] = sblocks[order[k]];
+    std::stable_sort(places.begin(), places.end(),
+                     [](const SumPlace& x, const SumPlace& y) { return x.work > y.work; });
+    p.sblocks.reserve(places.size());
+    for (const SumPlace& k : places) {
+        const SimDesc& s = sims[k.sim];
+        p.sblocks.push_back(sum_block(s, k.sim, k.q0, B, W, rows[s.row0 + k.q0 / B]));
+    }
     // Longest first (VALU ops per lane and j: R*15+6; a diagonal task's
     // block m passes over m + 1 of the row's sub-blocks).
     auto cost = [&](const MutualTask& t) {
