@@ -406,9 +406,12 @@ static long long group_slab_entries(long long gn, long long nrows, int B, int W)
 // longest task of every run of 256 (eight simulations of 4,000 to 18,600
 // particles, 1,097 workgroups: the fullest CU holds 1.26 times the mean).
 // Every second run is reversed, so long tasks meet short ones (1.06 times;
-// their step takes 222 us instead of 245).  Longer lists stay longest first:
-// their workgroups are dealt out as others end.  per_wg tasks make a
-// workgroup; a last one with fewer keeps its place.
+// their step takes 222 us instead of 245).  Lists beyond kTailPieces
+// workgroups, the grouped kernel's residents, stay longest first: its
+// workgroups are then dealt out as others end.  (k_mutual with R = 4 holds
+// more at once, so its lists of 1,541 workgroups and over, from 20,000
+// particles on, are in order of size though still one round.)  per_wg tasks
+// make a workgroup; a last one with fewer keeps its place.
 template <typename T>
 static void deal_out(std::vector<T>& tasks, int per_wg) {
     const size_t run = 256 * (size_t)per_wg, n = tasks.size() / per_wg * per_wg;
@@ -1514,10 +1517,13 @@ static int launch_step_run(hipGraphExec_t one, hipGraphExec_t many, int count, h
 
 // Before graphs are captured and launched on st: a plan just made is waited
 // for, so that its uploads are complete before they are captured around, and
-// so is the work before a run of steps on a stream of the caller's.  On the
-// default stream a run of steps queues behind the work before it (waiting for
-// it at each call, and running the graphs on the capture stream between two
-// events, held a call of 16 steps of 2,048 particles 40 us longer, of 168).
+// so is the work before a run of steps on a stream of the caller's, which a
+// caller may destroy as soon as it has waited for it: at most one call's
+// graphs, each with a fork to the library's own stream, are under way there.
+// On the default stream a run of steps queues behind the work before it
+// (waiting for it at each call, and running the graphs on the capture stream
+// between two events, held a call of 16 steps of 2,048 particles 40 us longer,
+// of 168).
 static int settle_plan(hipStream_t st, bool replanned) {
     if (replanned || st) GI_HIP(hipStreamSynchronize(st));
     return 0;

@@ -60,7 +60,9 @@ struct GroupTask {
 // 64 / R i-particles from i0 on of simulation sim in the direct pass (the
 // last block of a simulation may be ragged), with the simulation's ranges
 // beside them, and how many wavefronts of a workgroup take iron j: a
-// workgroup starts from one load, not two in turn, and divides nothing.
+// workgroup starts from one load, not two in turn, and divides nothing.  A
+// workgroup of the energy pass takes an entry, one of the force eight
+// i-particles of it.
 struct DirectBlock {
     int sim, i0, start, fe_end, end, iron_waves, pad0, pad1;
 };

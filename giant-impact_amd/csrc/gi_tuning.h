@@ -165,9 +165,9 @@ inline long long batched_piece_len(long long n, long long L0) {
 
 // The row for a launch of ntot particles.  Several simulations in one launch
 // (the separate bodies) have the work of one with as many pairs, sum n^2,
-// and are placed by that size: two of 8,000 (11,314) step in 59 us by the
-// direct pass's row and in 66 by the row of 16,000; two of 18,000 (25,456)
-// in 140 and, by the row of 36,000, 159.
+// and are placed by that size: two of 6,200 (8,768) and two of 8,000 (11,314)
+// step in 43 and 58 us by the direct pass's rows, in 55 and 66 by the rows of
+// 12,400 and 16,000.
 inline Tiling choose_tiling(long long ntot, long long pairs, int nsims) {
     if (tiling_override().active) return tiling_override().t;
     if (nsims > 1) ntot = (long long)std::ceil(std::sqrt((double)pairs));

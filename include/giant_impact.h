@@ -30,7 +30,9 @@
  * Code/CommonCode/commonFunctions.h:12-22.)
  *
  * Streams: a gi_stream_t is a hipStream_t; NULL means the default stream.
- * Work is enqueued asynchronously in stream order.  Scratch buffers are owned
+ * Work is enqueued asynchronously in stream order (gi_impact_steps,
+ * gi_impact_steps_float_recenter and gi_separate_steps first wait for the work
+ * before them on a stream that is not the default one).  Scratch buffers are owned
  * by the library, one set per device, grown on demand and reused; calls that
  * overlap on one device from several host threads or streams are not
  * supported (the reference is single-threaded, one default stream).
