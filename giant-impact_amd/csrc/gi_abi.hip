@@ -1129,12 +1129,19 @@ static int launch_gravity(DevCtx* ctx, Workspace* ws, const float4* pos, bool po
     return 0;
 }
 
+// log2 of the workgroups of k_direct that share a block table entry of
+// 64 / lanes i-particles.
+static int direct_per_log2(int lanes) {
+    int per_log2 = 0;
+    while ((kDirectI << per_log2) * lanes < 64) ++per_log2;
+    return per_log2;
+}
+
 // k_direct over a block table of 64 / lanes i-particles per entry.
 template <int MOVE>
 static void direct_kernel(int lanes, int nblocks, hipStream_t st, const float4* pos, const float4* vel,
                           const DirectBlock* blocks, const SimDesc* sims, float4* force, const FusedMove& mv) {
-    int per_log2 = 0;
-    while ((kDirectI << per_log2) * lanes < 64) ++per_log2;
+    const int per_log2 = direct_per_log2(lanes);
     hipLaunchKernelGGL(k_direct<MOVE>, dim3((unsigned)nblocks << per_log2), dim3(64 * kDirectForceWaves), 0, st, pos,
                        vel, blocks, per_log2, sims, force, mv);
 }
@@ -1725,7 +1732,7 @@ int gi_plan_info(int* mutual, int* r, long long* pair_tasks, long long* chunk_le
     if (r) *r = valid ? p.tiling.R : 0;
     if (pair_tasks)
         *pair_tasks = !valid     ? 0
-                      : p.direct ? (long long)p.dblocks.size()
+                      : p.direct ? (long long)p.dblocks.size() << direct_per_log2(p.direct_lanes)
                                  : (long long)(p.tasks.size() + (p.group_rows > 1 ? p.gtasks.size() : p.mtasks.size()));
     if (chunk_len) *chunk_len = valid ? p.chunk_len : 0;
     return 0;
